@@ -19,8 +19,10 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
+#include "cg_resident.hpp"
 #include "krylov.hpp"
 
 namespace frehg {
@@ -1052,7 +1054,12 @@ Krylov::Krylov(const Geo& g, bool three_d, hipStream_t stream, Profiler* prof, c
   part_ = ws.part;
   part_u_ = ws.part_u;
   ctl_ = ws.ctl;
-  host_ctl_ = &host_ctl_own_;
+  host_ctl_ = host_ctl_own_;
+  // the resident solve needs none of the CG vectors: its exchange buffers take their place
+  double* words[4] = {r_, z_, p0_, p1_};
+  for (int q = 0; q < 4; ++q) halo_[q] = reinterpret_cast<unsigned long long*>(words[q]);
+  mail_ = reinterpret_cast<unsigned long long*>(q_);
+  if (plan_[0].nblk > 1 && 2 * (size_t)plan_[0].nblk * kCgMailWords > (size_t)n_) plan_[0] = ResidentPlan{};
   // no autotuning (it would time launches with events): two columns per lane, whole columns per
   // block in 3D, unless FREHG_SPMV_SHAPE pins a shape
   if (!tuned_[0]) {
@@ -1127,6 +1134,93 @@ void Krylov::setup_shapes() {
       tuned_[prec] = true;
     }
   }
+  setup_resident();
+}
+
+// Tiling of the resident CG solve: a solve of up to 2048 rows takes one block (no exchange), a larger one
+// the fewest cells per thread (1, 2, 4, 8) whose tiles number at most one per compute unit, and of those the
+// tiling with the least halo and blocks. Operators beyond eight cells per thread (4096 rows per compute
+// unit, fewer where the LDS is short) stream: there an iteration is bound by HBM, not by latency.
+// us per iteration on MI355X, streaming (at the shapes the solver chose) and resident:
+//   rows    819   4096   8000   80000  131072  262144 (3D)  512000  589824 | 2D: 2400  16384  262144  360000
+//   stream  28.1  34.7   40.0   67.7   51.6    90.0         93.3    75.7   |     20.5  20.4   25.4    28.7
+//   here     1.5   3.2    3.4    3.7    3.8     4.5          5.7     9.0   |      2.7   3.4    3.7     4.2
+Krylov::ResidentPlan Krylov::resident_plan(const Geo& g, bool three_d, size_t elt, int max_blocks, size_t max_lds) {
+  ResidentPlan best;
+  const int nx = g.nx, ny = g.ny, nz = three_d ? g.nz : 1;
+  const long long cells = (long long)nx * ny * nz;
+  // p with its halo; with eight cells per thread also D and the couplings (see k_cg_resident)
+  auto lds = [&](int cpt, long long tx, long long ty, long long tz) {
+    long long n = (tx + 2) * (ty + 2) * (three_d ? tz + 2 : 1);
+    if (cpt == 8) n += tx * ty * tz + (tx + 1) * ty * tz + tx * (ty + 1) * tz + (three_d ? tx * ty * (tz + 1) : 0);
+    return (size_t)n * elt;
+  };
+  auto fits = [&](int cpt, int tx, int ty, int tz) {
+    return lds(cpt, tx, ty, tz) <= std::min(max_lds, (size_t)(cpt == 8 ? kCgMaxLdsOp : kCgMaxLds));
+  };
+  auto take = [&](int cpt, int tx, int ty, int tz) {
+    best.cpt = cpt;
+    best.tx = tx;
+    best.ty = ty;
+    best.tz = tz;
+    best.ntx = (int)ceil_div(nx, tx);
+    best.nty = (int)ceil_div(ny, ty);
+    best.ntz = (int)ceil_div(nz, tz);
+    best.nblk = (unsigned int)(best.ntx * best.nty * best.ntz);
+    best.lds = lds(cpt, tx, ty, tz);
+  };
+  for (int cpt = 1; cpt <= 4; cpt *= 2)
+    if (cells <= (long long)kCgNT * cpt && fits(cpt, nx, ny, nz)) {
+      take(cpt, nx, ny, nz);
+      return best;
+    }
+  const int most = std::min(max_blocks, kCgMaxBlocks);
+  for (int cpt = 1; cpt <= 8; cpt *= 2) {
+    const long long cap = (long long)kCgNT * cpt;
+    if (cells > cap * most) continue;
+    long long least = -1;
+    for (int px = 1; px <= std::min(nx, most); ++px) {
+      const int tx = (int)ceil_div(nx, px);
+      if ((int)ceil_div(nx, tx) != px || tx > cap) continue;
+      for (int py = 1; py <= std::min(ny, most / px); ++py) {
+        const int ty = (int)ceil_div(ny, py);
+        if ((int)ceil_div(ny, ty) != py || (long long)tx * ty > cap) continue;
+        int tz = (int)std::min<long long>(nz, cap / ((long long)tx * ty));
+        // (eight cells per thread: layers as the LDS allows)
+        while (tz > 1 && !fits(cpt, tx, ty, tz)) --tz;
+        const int pz = (int)ceil_div(nz, tz);
+        if ((long long)px * py * pz > most) continue;
+        tz = (int)ceil_div(nz, pz);
+        const long long halo = 2LL * (ty * tz + tx * tz + (three_d ? tx * ty : 0));
+        if (halo > (long long)kCgNT * kCgHalo || !fits(cpt, tx, ty, tz)) continue;
+        // few halo values, and few blocks to wait for
+        const long long cost = halo + 2LL * px * py * pz;
+        if (least < 0 || cost < least) {
+          least = cost;
+          take(cpt, tx, ty, tz);
+        }
+      }
+    }
+    if (least >= 0) return best;
+  }
+  return best;
+}
+
+void Krylov::setup_resident() {
+  if (tuned_[0]) return;  // a pinned SpMV shape asks for the streaming solver
+  int cus = 0, lds = 0;
+  if (hipGetDevice(&device_) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device_) != hipSuccess ||
+      hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device_) != hipSuccess || cus < 1) {
+    (void)hipGetLastError();
+    return;
+  }
+  for (int prec = 0; prec < 2; ++prec) plan_[prec] = resident_plan(g_, three_d_, prec ? 4 : 8, cus, (size_t)std::max(0, lds - 2048));
+}
+
+void Krylov::clear_exchange() {
+  for (unsigned long long* h : halo_) FREHG_HIP(hipMemsetAsync(h, 0, (size_t)n_ * sizeof(unsigned long long), s_));
+  FREHG_HIP(hipMemsetAsync(mail_, 0, mail_words_ * sizeof(unsigned long long), s_));
 }
 
 void Krylov::build() {
@@ -1140,7 +1234,14 @@ void Krylov::build() {
   }
   FREHG_HIP(hipMalloc(&ctl_, 3 * sizeof(KrylovCtl)));
   FREHG_HIP(hipMemsetAsync(ctl_, 0, 3 * sizeof(KrylovCtl), s_));
-  FREHG_HIP(hipHostMalloc(&host_ctl_, sizeof(KrylovCtl), hipHostMallocDefault));
+  FREHG_HIP(hipHostMalloc(&host_ctl_, 2 * sizeof(KrylovCtl), hipHostMallocDefault));
+  const unsigned int nblk = std::max(plan_[0].nblk, plan_[1].nblk);
+  if (nblk > 1) {
+    mail_words_ = 2 * (size_t)nblk * kCgMailWords;
+    for (unsigned long long*& h : halo_) FREHG_HIP(hipMalloc(&h, (size_t)n_ * sizeof(unsigned long long)));
+    FREHG_HIP(hipMalloc(&mail_, mail_words_ * sizeof(unsigned long long)));
+    clear_exchange();
+  }
   FREHG_HIP(hipStreamSynchronize(s_));
 }
 
@@ -1152,7 +1253,7 @@ void Krylov::release() {
                   (void*)r32_, (void*)z32_, (void*)p032_, (void*)p132_, (void*)q32_, (void*)d32_,
                   (void*)rh_, (void*)v0_, (void*)v1_, (void*)sv_, (void*)tv_, (void*)rh32_, (void*)v032_,
                   (void*)v132_, (void*)sv32_, (void*)tv32_, (void*)part_, (void*)part_u_, (void*)ctl_,
-                  (void*)stage_})
+                  (void*)stage_, (void*)halo_[0], (void*)halo_[1], (void*)halo_[2], (void*)halo_[3], (void*)mail_})
     if (p) (void)hipFree(p);
   if (host_ctl_) (void)hipHostFree(host_ctl_);
 }
@@ -1354,17 +1455,23 @@ int Krylov::cg_finish(const StencilView<T>& A, T* x, T* r, T* z, T* p0, T* p1, T
   }
   // a solve from an uncleared x0 = 0 that ended before its first update
   if (x_fresh && host_ctl_->iters == 0) zero_interior<T>(x, nullptr);
+  const int iters = cg_outcome<T>(res_norm, rhs_norm, converged);
+  // each launched 3D iteration recorded one spmv and one update launch
+  if (three_d_ && launched > iters) {
+    prof_->discard_last(kt_spmv, (size_t)(launched - iters));
+    prof_->discard_last(FREHG_KT_GW_UPDATE, (size_t)(launched - iters));
+  }
+  return iters;
+}
+
+template <typename T>
+int Krylov::cg_outcome(double* res_norm, double* rhs_norm, bool* converged) {
   if (host_ctl_->breakdown)
     throw ConvergenceError(std::string("Krylov ") + (three_d_ ? "3D" : "2D") + (sizeof(T) == 4 ? " fp32" : " fp64") +
                            ": breakdown (p.Ap = " + std::to_string(host_ctl_->pq) + " at iteration " +
                            std::to_string(host_ctl_->iters + 1) + ", ||D^-1 r||^2 = " + std::to_string(host_ctl_->zz) +
                            ")");
   const int iters = host_ctl_->iters;
-  // each launched 3D iteration recorded one spmv and one update launch
-  if (three_d_ && launched > iters) {
-    prof_->discard_last(kt_spmv, (size_t)(launched - iters));
-    prof_->discard_last(FREHG_KT_GW_UPDATE, (size_t)(launched - iters));
-  }
   if (sizeof(T) == 8) last_iters_ = iters;
   else last_inner_iters_ = iters;
   *res_norm = std::sqrt(host_ctl_->zz);
@@ -1373,11 +1480,90 @@ int Krylov::cg_finish(const StencilView<T>& A, T* x, T* r, T* z, T* p0, T* p1, T
   return iters;
 }
 
+namespace {
+// Launches of the resident solver with more than one block wait for one another's blocks, so two of
+// them (on two contexts' streams) must not share a device: each holds its device's lock until it is done.
+constexpr int kMaxDevices = 64;
+std::mutex g_resident_mu[kMaxDevices];
+
+template <typename T, bool THREE_D>
+void launch_resident(int cpt, unsigned int nblk, size_t lds, hipStream_t s, const CgResidentArgs<T>& a) {
+  switch (cpt) {
+    case 1: hipLaunchKernelGGL((k_cg_resident<T, THREE_D, 1>), dim3(nblk), dim3(kCgNT), lds, s, a); break;
+    case 2: hipLaunchKernelGGL((k_cg_resident<T, THREE_D, 2>), dim3(nblk), dim3(kCgNT), lds, s, a); break;
+    case 4: hipLaunchKernelGGL((k_cg_resident<T, THREE_D, 4>), dim3(nblk), dim3(kCgNT), lds, s, a); break;
+    default: hipLaunchKernelGGL((k_cg_resident<T, THREE_D, 8>), dim3(nblk), dim3(kCgNT), lds, s, a);
+  }
+  FREHG_LAUNCH_CHECK();
+}
+}  // namespace
+
+template <typename T>
+bool Krylov::cg_resident(const StencilView<T>& A, const T* b, const T* bn, T* x, const unsigned char* fixed, bool zero,
+                         bool guard, double rtol, double atol, int max_it, const T* r0, const KrylovCtl* started) {
+  const ResidentPlan& pl = plan_[sizeof(T) == 4 ? 1 : 0];
+  std::unique_lock<std::mutex> lock;
+  if (pl.nblk > 1) lock = std::unique_lock<std::mutex>(g_resident_mu[device_ % kMaxDevices]);
+  if (++launch_ >= (1u << 20)) {  // the tags start again: no old one may be left
+    launch_ = 1;
+    if (mail_words_) clear_exchange();
+  }
+  CgResidentArgs<T> a;
+  a.g = g_;
+  a.A = A;
+  a.b = b;
+  a.bn = bn;
+  a.x = x;
+  a.fixed = fixed;
+  a.r0 = r0;
+  a.ctl = started;
+  // the outcome goes straight to pinned host memory (a borrowed workspace has none: copied below)
+  KrylovCtl* out = borrowed_ ? ctl_ : host_ctl_;
+  host_ctl_[1].iters = 0;
+  a.out = out;
+  a.timeout = &out[1].iters;
+  a.rtol = rtol;
+  a.atol = atol;
+  a.max_it = max_it;
+  a.guard = guard ? 1 : 0;
+  a.x0_zero = zero ? 1 : 0;
+  a.tx = pl.tx;
+  a.ty = pl.ty;
+  a.tz = pl.tz;
+  a.ntx = pl.ntx;
+  a.nty = pl.nty;
+  a.ntz = pl.ntz;
+  for (int h = 0; h < 2; ++h) {
+    a.lo[h] = halo_[h];
+    a.hi[h] = halo_[2 + h];
+  }
+  a.mail = mail_;
+  a.launch = launch_;
+  if (three_d_) launch_resident<T, true>(pl.cpt, pl.nblk, pl.lds, s_, a);
+  else launch_resident<T, false>(pl.cpt, pl.nblk, pl.lds, s_, a);
+  if (borrowed_) FREHG_HIP(hipMemcpyAsync(host_ctl_, ctl_, 2 * sizeof(KrylovCtl), hipMemcpyDeviceToHost, s_));
+  FREHG_HIP(hipStreamSynchronize(s_));
+  if (host_ctl_[1].iters == 0) return true;
+  plan_[0] = plan_[1] = ResidentPlan{};
+  return false;
+}
+
 template <typename T>
 int Krylov::run_pcg(const StencilView<T>& A, const T* b, const T* bn, T* x, const unsigned char* fixed,
                     bool x0_zero, bool guard, double rtol, double atol, int max_it, KrylovCtl* ctl,
                     T* r, T* z, T* p0, T* p1, T* q, bool* rejected, double* res_norm,
                     double* rhs_norm, bool* converged, int kt_spmv) {
+  *rejected = false;
+  if (resident(sizeof(T) == 4 ? 1 : 0)) {
+    bool ok = cg_resident<T>(A, b, bn, x, fixed, x0_zero, guard, rtol, atol, max_it, nullptr, nullptr);
+    if (ok && host_ctl_->guess_rejected) {
+      *rejected = true;
+      ok = cg_resident<T>(A, b, bn, x, fixed, true, guard, rtol, atol, max_it, nullptr, nullptr);
+    }
+    if (ok) return cg_outcome<T>(res_norm, rhs_norm, converged);
+    if (borrowed_)  // the exchange buffers become CG vectors again (finite at every entry)
+      for (double* v : {r_, z_, p0_, p1_, q_}) FREHG_HIP(hipMemsetAsync(v, 0, (size_t)n_ * sizeof(double), s_));
+  }
   cg_start<T>(A, b, bn, x, fixed, x0_zero, guard, rtol, atol, max_it, ctl, r, z, p0);
   *rejected = false;
   bool zero = x0_zero;
@@ -1395,30 +1581,6 @@ int Krylov::run_pcg(const StencilView<T>& A, const T* b, const T* bn, T* x, cons
   cg_iterations<T>(A, x, r, z, p0, p1, q, ctl, 0, batch, kt_spmv, fresh);
   return cg_finish<T>(A, x, r, z, p0, p1, q, ctl, max_it, batch, batch, res_norm, rhs_norm, converged, kt_spmv,
                       fresh);
-}
-
-void Krylov::enqueue_cg(const StencilView<double>& A, const double* b, const double* bn, double* x,
-                        const unsigned char* fixed, bool x0_zero, const KrylovConfig& cfg, int budget) {
-  if (cfg.ksp != FREHG_KSP_CG || cfg.precision != 0) throw ArgError("Krylov::enqueue_cg: FP64 CG only");
-  if (three_d_ && !tuned_[0]) throw ArgError("Krylov::enqueue_cg: 3D SpMV shape not tuned yet");
-  cg_start<double>(A, b, bn, x, fixed, x0_zero, false, cfg.rtol, cfg.atol, cfg.max_it, ctl_, r_, z_, p0_);
-  enq_fresh_ = x0_zero && fixed == nullptr;
-  cg_iterations<double>(A, x, r_, z_, p0_, p1_, q_, ctl_, 0, budget, three_d_ ? FREHG_KT_GW_SPMV : FREHG_KT_SW_SPMV,
-                        enq_fresh_);
-}
-
-SolveResult Krylov::finish_cg(const StencilView<double>& A, double* x, const KrylovConfig& cfg, int budget) {
-  SolveResult res;
-  bool conv = false;
-  res.iterations = cg_finish<double>(A, x, r_, z_, p0_, p1_, q_, ctl_, cfg.max_it, budget, budget,
-                                     &res.residual_norm, &res.rhs_norm, &conv,
-                                     three_d_ ? FREHG_KT_GW_SPMV : FREHG_KT_SW_SPMV, enq_fresh_);
-  res.converged = conv;
-  if (!conv)
-    throw ConvergenceError(std::string("Krylov ") + (three_d_ ? "3D" : "2D") + ": not converged within max_it (" +
-                           std::to_string(res.iterations) + " iterations, ||D^-1 r|| = " +
-                           std::to_string(res.residual_norm) + ", ||D^-1 b|| = " + std::to_string(res.rhs_norm) + ")");
-  return res;
 }
 
 template <typename T>
@@ -1551,7 +1713,8 @@ SolveResult Krylov::solve(const StencilView<double>& A, const StencilView<float>
                           bool guard_guess, const KrylovConfig& cfg, unsigned int swept_blocks) {
   SolveResult res;
   // (the autotuner's SpMV launches write part_, which holds a caller's sweep partials)
-  if (!tuned_[0] && !swept_blocks) autotune<double>(A);
+  const bool streams = cfg.ksp != FREHG_KSP_CG || !resident(cfg.precision == 0 || A32 == nullptr ? 0 : 1);
+  if (streams && !tuned_[0] && !swept_blocks) autotune<double>(A);
   if (swept_blocks && (cfg.precision == 0 || A32 == nullptr))
     throw ArgError("Krylov: a pre-swept solve is a mixed-precision solve");
   if (cfg.precision == 0 || A32 == nullptr) {
@@ -1633,7 +1796,7 @@ SolveResult Krylov::solve(const StencilView<double>& A, const StencilView<float>
     hipLaunchKernelGGL(k_fin_refine, dim3(1), dim3(kRedThreads), 0, s_, (const double*)stage_, kRedStage, outer, 1,
                        cfg.rtol, cfg.atol, guard_guess ? 1 : 0, inner, cfg.inner_rtol, cfg.max_it);
     FREHG_LAUNCH_CHECK();
-    if (!tuned_[0]) autotune<double>(A);
+    if (streams && !tuned_[0]) autotune<double>(A);
   } else {
     refine(x, nullptr, xw_, true);
   }
@@ -1648,7 +1811,7 @@ SolveResult Krylov::solve(const StencilView<double>& A, const StencilView<float>
   res.residual_norm = std::sqrt(host_ctl_->zz);
   bool conv = host_ctl_->converged != 0;
   const StencilView<float> A32v = *A32;
-  if (!tuned_[1]) autotune<float>(A32v);
+  if (streams && !tuned_[1]) autotune<float>(A32v);
   while (!conv && res.refinements < cfg.max_refine) {
     bool rej = false, iconv = false;
     double rn = 0, bnrm = 0;
@@ -1658,10 +1821,15 @@ SolveResult Krylov::solve(const StencilView<double>& A, const StencilView<float>
     const double inner_rt = std::min(0.5, std::max(cfg.inner_rtol, 0.5 * gap));
     if (fused) {
       // started by the sweep (same tolerance, computed on the device)
+      if (resident(1) && cg_resident<float>(A32v, nullptr, nullptr, d32_, nullptr, true, false, 0.0, 0.0, cfg.max_it,
+                                            r32_, inner)) {
+        res.iterations += cg_outcome<float>(&rn, &bnrm, &iconv);
+      } else {
       const int batch = std::max(2, last_inner_iters_ + 1);
       cg_iterations<float>(A32v, d32_, r32_, z32_, p032_, p132_, q32_, inner, 0, batch, FREHG_KT_GW_SPMV32, true);
       res.iterations += cg_finish<float>(A32v, d32_, r32_, z32_, p032_, p132_, q32_, inner, cfg.max_it, batch, batch,
                                          &rn, &bnrm, &iconv, FREHG_KT_GW_SPMV32, true);
+      }
     } else {
       res.iterations += run<float>(cfg.ksp, A32v, b32_, nullptr, d32_, fixed, true, false, inner_rt, 0.0,
                                    cfg.max_it, inner, &rej, &rn, &bnrm, &iconv,

@@ -122,14 +122,6 @@ class Krylov {
   };
   SweepTarget first_sweep_target();
 
-  // FP64 CG split for graph capture: enqueue_cg queues the start and `budget` iterations without
-  // any host synchronisation; finish_cg (same budget) waits, continues past the budget if needed
-  // and returns the result as solve() would (x0 = 0 or x, no guess guard).
-  void enqueue_cg(const StencilView<double>& A, const double* b, const double* bn, double* x,
-                  const unsigned char* fixed, bool x0_zero, const KrylovConfig& cfg, int budget);
-  SolveResult finish_cg(const StencilView<double>& A, double* x, const KrylovConfig& cfg, int budget);
-  int last_iterations() const { return last_iters_; }
-
   // CG SpMV launch shape per precision (0 FP64, 1 FP32): cells per lane (1: one column per
   // thread on 64 x 4 tiles; 2: two adjacent columns per lane on 128 x 4 tiles, paired aligned
   // loads, x-neighbours by wave shifts) and layers per block of the z-march (kc).
@@ -145,8 +137,30 @@ class Krylov {
   template <typename T>
   void autotune(const StencilView<T>& A);
   bool tuned(int prec) const { return tuned_[prec]; }
+  // Tiling of the resident CG solve (cg_resident.hpp) for this grid, if it has one: cells per thread
+  // (0: the solve streams), cells per tile, tiles, blocks and dynamic LDS bytes.
+  struct ResidentPlan {
+    int cpt = 0;
+    int tx = 1, ty = 1, tz = 1, ntx = 1, nty = 1, ntz = 1;
+    unsigned int nblk = 0;
+    size_t lds = 0;
+  };
+  static ResidentPlan resident_plan(const Geo& g, bool three_d, size_t elt, int max_blocks, size_t max_lds);
+  bool resident(int prec) const { return plan_[prec].cpt > 0; }
+  unsigned int resident_blocks(int prec) const { return plan_[prec].nblk; }  // 0: the solve streams
 
  private:
+  void setup_resident();
+  void clear_exchange();
+  // Solves by one launch of the resident kernel and waits for it; the outcome is in host_ctl_. False when a
+  // wait inside the launch ran out (x may hold a mixture of iterates; the instance then streams).
+  // r0 / started: a solve begun by a refinement sweep (x0 = 0).
+  template <typename T>
+  bool cg_resident(const StencilView<T>& A, const T* b, const T* bn, T* x, const unsigned char* fixed, bool zero,
+                   bool guard, double rtol, double atol, int max_it, const T* r0, const KrylovCtl* started);
+  // Errors, counters and norms of a finished CG solve from host_ctl_.
+  template <typename T>
+  int cg_outcome(double* res_norm, double* rhs_norm, bool* converged);
   void setup_shapes();
   void build();
   void release();
@@ -192,7 +206,6 @@ class Krylov {
   int kc_f_ = 1;
   dim3 grid_f_;
   unsigned int nb_f_ = 0, part_cap_ = 0;
-  bool enq_fresh_ = false;  // enqueue_cg started from an uncleared x0 = 0
   // CG update: 128 x 4 tiles of cell pairs, kc_u_ layers per block; its partials (r.z, z.z)
   int kc_u_ = 1;
   dim3 grid_u_;
@@ -211,7 +224,12 @@ class Krylov {
   KrylovCtl* ctl_ = nullptr;  // [0] main / outer, [1] inner
   KrylovCtl* host_ctl_ = nullptr;
   bool borrowed_ = false;  // workspace owned by the caller (no allocation, no autotuning)
-  KrylovCtl host_ctl_own_{};  // host mirror of the control block in borrowed mode
+  KrylovCtl host_ctl_own_[2] = {};  // host mirrors of the control blocks in borrowed mode
+  ResidentPlan plan_[2];          // resident CG solve per precision (0 FP64, 1 FP32)
+  int device_ = 0;
+  unsigned int launch_ = 0;       // resident launches of this instance (the tag of their exchanges)
+  unsigned long long *halo_[4] = {}, *mail_ = nullptr;  // its exchange buffers: low, low, high, high words; sums
+  size_t mail_words_ = 0;
   int last_iters_ = 8;
   int last_inner_iters_ = 8;
   int last_bcg_iters_ = 8;

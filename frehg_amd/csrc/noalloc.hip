@@ -15,6 +15,7 @@
 // CG vectors and writes every entry of the padded operator, and calls that overlap on one GPU
 // (two host threads, or two processes) race. Host threads of one process are serialised by a
 // per-device lock.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -40,8 +41,10 @@ std::mutex g_call_mu[kMaxDevices];      // serialises this process's calls per d
 
 constexpr int NT = 256;
 
-// Fill kernel (no hipMemsetAsync, so a caller may also capture the call's launches).
-__global__ __launch_bounds__(NT) void k_na_zero(double* a, long long n) {
+// Fill kernel (no hipMemsetAsync, so a caller may also capture the call's launches): the CG vectors or
+// exchange buffers, and the flag word.
+__global__ __launch_bounds__(NT) void k_na_zero(double* a, long long n, int* flags) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *flags = 0;
   for (long long c = (long long)blockIdx.x * NT + threadIdx.x; c < n; c += (long long)gridDim.x * NT) a[c] = 0.0;
 }
 
@@ -169,14 +172,16 @@ void ls_solve_noalloc(int device, hipStream_t s, int ndim, int nx, int ny, int n
   double* x = reinterpret_cast<double*>(take((size_t)n * sizeof(double)));
   int* flags = reinterpret_cast<int*>(take(sizeof(int)));
   const KrylovWorkspace ws = Krylov::carve_workspace(base, g, three);
-  // CG vectors from earlier calls hold other geometries: clear them (their ghost entries meet
-  // zero coefficients and must be finite), and the flag word.
-  const unsigned zb = (unsigned)std::min<long long>(4096, (n + NT - 1) / NT);
-  for (double* v : {ws.r, ws.z, ws.p0, ws.p1, ws.q}) {
-    hipLaunchKernelGGL(k_na_zero, dim3(zb), dim3(NT), 0, s, v, n);
-    FREHG_LAUNCH_CHECK();
-  }
-  hipLaunchKernelGGL(k_na_zero, dim3(1), dim3(NT), 0, s, reinterpret_cast<double*>(flags), 1LL);
+  Profiler off;  // no timing events (they would be created on first use)
+  Krylov kry(g, three, s, &off, ws);
+  // CG vectors from earlier calls hold other geometries: clear them (their ghost entries meet zero
+  // coefficients and must be finite; for the resident solve, which keeps its vectors on the compute
+  // units, they are exchange buffers whose words must not carry a tag) with the control blocks behind
+  // them, and the flag word. A resident solve of one block exchanges nothing.
+  double* z0 = kry.resident_blocks(0) == 1 ? reinterpret_cast<double*>(ws.ctl) : ws.r;
+  const long long zn = (reinterpret_cast<char*>(ws.ctl + 3) - reinterpret_cast<char*>(z0)) / (long long)sizeof(double);
+  hipLaunchKernelGGL(k_na_zero, dim3((unsigned)std::min<long long>(4096, (zn + NT - 1) / NT)), dim3(NT), 0, s, z0, zn,
+                     flags);
   FREHG_LAUNCH_CHECK();
   NaOperator op{};
   op.diag = diag;
@@ -190,8 +195,6 @@ void ls_solve_noalloc(int device, hipStream_t s, int ndim, int nx, int ny, int n
   FREHG_HIP(hipStreamSynchronize(s));
   if (hflags & 2) throw ArgError("frehg_ls_solve_noalloc: zero diagonal (Jacobi needs D != 0)");
   if (hflags & 1) throw ArgError("frehg_ls_solve_noalloc: operator is not symmetric (CG requires A = A^T)");
-  Profiler off;  // no timing events (they would be created on first use)
-  Krylov kry(g, three, s, &off, ws);
   const StencilView<double> A{D, ax, ay, az};
   const SolveResult sr = kry.solve(A, nullptr, b, nullptr, x, nullptr, true, false, kc);
   const long long rows = (long long)nx * ny * (three ? nz : 1);

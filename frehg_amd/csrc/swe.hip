@@ -723,32 +723,18 @@ void SweState::copy_field(const double* src, double* dst) {
   FREHG_LAUNCH_CHECK();
 }
 
-// With FREHG_SW_GRAPH=1 the step's kernels are replayed from two captured graphs around the
-// surface solve (its start and a budget of CG iterations are in the first): a graph launch
-// replaces a host launch per kernel of this launch-bound 2D step. The graphs are captured again
-// when the parameters, the forcing or the budget change; iterations past the budget run eagerly
-// (Krylov::finish_cg). Off by default: on the 512 x 512 coupled workload the replayed kernels
-// run back to back but the graph is dispatched in segments separated by 10-40 us, and the step
-// is no faster than with eager launches.
+// With FREHG_SW_GRAPH=1 the step's kernels are replayed from two captured graphs, one on either side of
+// the surface solve: a graph launch replaces a host launch per kernel of this launch-bound 2D step. The
+// graphs are captured again when the parameters or the forcing change. Off by default: on the 512 x 512
+// coupled workload the replayed kernels run back to back but the graph is dispatched in segments
+// separated by 10-40 us, and the step is no faster than with eager launches.
 void SweState::step(double rain, double evap, frehg_solve_stats* st) {
   KrylovConfig kc = krylov_config(p_.solver, "frehg_swe_step");
   kc.precision = 0;  // the surface system is small; it stays FP64
   StencilView<double> A{f_["Sct"], ax_, ay_, nullptr};
   SolveResult sr;
-  if (use_graph_ && kc.ksp == FREHG_KSP_CG && solved_) {
-    // budget: one iteration more than the last solve took; grown at once, shrunk only after it
-    // has been too large for 16 steps (each change costs a capture)
-    const int want = std::max(2, kry_->last_iterations() + 1);
-    if (budget_ == 0 || want > budget_) {
-      budget_ = want;
-      shrink_ = 0;
-    } else if (want < budget_ && ++shrink_ >= 16) {
-      budget_ = want;
-      shrink_ = 0;
-    } else if (want == budget_) {
-      shrink_ = 0;
-    }
-    const bool same = graph_pre_ && graph_rain_ == rain && graph_evap_ == evap && graph_budget_ == budget_ &&
+  if (use_graph_) {
+    const bool same = graph_pre_ && graph_rain_ == rain && graph_evap_ == evap &&
                       std::memcmp(&graph_params_, &p_, sizeof(p_)) == 0;
     if (!same) {
       for (hipGraphExec_t* ge : {&graph_pre_, &graph_post_})
@@ -769,25 +755,19 @@ void SweState::step(double rain, double evap, frehg_solve_stats* st) {
         FREHG_HIP(hipGraphInstantiate(out, g, nullptr, nullptr, 0));
         FREHG_HIP(hipGraphDestroy(g));
       };
-      capture(&graph_pre_, [&] {
-        enq_pre(evap);
-        kry_->enqueue_cg(A, b_, f_["Srhs"], f_["eta"], fixed_, true, kc, budget_);
-      });
+      capture(&graph_pre_, [&] { enq_pre(evap); });
       capture(&graph_post_, [&] { enq_post(rain, evap); });
       graph_rain_ = rain;
       graph_evap_ = evap;
-      graph_budget_ = budget_;
       graph_params_ = p_;
     }
     FREHG_HIP(hipGraphLaunch(graph_pre_, s_));
-    sr = kry_->finish_cg(A, f_["eta"], kc, budget_);
-    FREHG_HIP(hipGraphLaunch(graph_post_, s_));
   } else {
     enq_pre(evap);
-    sr = kry_->solve(A, nullptr, b_, f_["Srhs"], f_["eta"], fixed_, true, false, kc);
-    enq_post(rain, evap);
-    solved_ = true;
   }
+  sr = kry_->solve(A, nullptr, b_, f_["Srhs"], f_["eta"], fixed_, true, false, kc);
+  if (use_graph_) FREHG_HIP(hipGraphLaunch(graph_post_, s_));
+  else enq_post(rain, evap);
   if (st) {
     std::memset(st, 0, sizeof(*st));
     st->iterations = sr.iterations;

@@ -80,11 +80,8 @@ class SweState {
   std::unique_ptr<Krylov> kry_;
   // captured step graphs (before / after the surface solve) and what they were captured for
   bool use_graph_ = false;  // FREHG_SW_GRAPH=1: replay the step from captured graphs
-  bool solved_ = false;  // the first step runs eagerly and sets the iteration estimate
-  int budget_ = 0, shrink_ = 0;
   hipGraphExec_t graph_pre_ = nullptr, graph_post_ = nullptr;
   double graph_rain_ = 0.0, graph_evap_ = 0.0;
-  int graph_budget_ = 0;
   frehg_swe_params graph_params_{};
 };
 

@@ -351,7 +351,8 @@ int frehg_profile_reset(frehg_ctx_t ctx);
  * FREHG_PREC_MIXED: the FP32 inner solve): cells per lane (1: one column per thread; 2: two
  * adjacent columns per lane with paired aligned loads) and layers per block. Set by the autotuner
  * at the first solve, or pinned by the environment variable FREHG_SPMV_SHAPE="cpl:kchunk" read at
- * frehg_re_init. No counterpart in the reference (PETSc's MatMult has no launch shape). */
+ * frehg_re_init. CG on operators of up to about a million rows runs whole in one launch instead (no
+ * SpMV launches, and none to time) unless a shape is pinned. No counterpart in the reference (PETSc's MatMult has no launch shape). */
 int frehg_spmv_shape(frehg_ctx_t ctx, int precision, int* cells_per_lane, int* kchunk);
 /* Streaming probe on `device`: the CG SpMV's HBM access mix (six FP64 reads and two FP64 writes
  * per cell, 16-byte accesses) with no neighbours and no reduction, over eight arrays of `cells`
