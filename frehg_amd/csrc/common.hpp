@@ -219,6 +219,10 @@ __global__ __launch_bounds__(256) inline void k_reduce_maxmin_stage(const double
 // out[0] = max of part[0..n) (floored at 0), out[1] = min of part[n..2n) (capped at 1e300);
 // tmp holds 2 * kRedStage doubles.
 inline void reduce_maxmin(const double* part, unsigned int n, double* tmp, double* out, hipStream_t s) {
+  if (n <= 2048) {  // (two loads per thread: one launch instead of two, 2.5 us each)
+    hipLaunchKernelGGL(k_reduce_maxmin, dim3(1), dim3(kRedThreads), 0, s, part, n, out);
+    return;
+  }
   hipLaunchKernelGGL(k_reduce_maxmin_stage, dim3(kRedStage), dim3(256), 0, s, part, n, tmp);
   hipLaunchKernelGGL(k_reduce_maxmin, dim3(1), dim3(kRedThreads), 0, s, (const double*)tmp, kRedStage, out);
 }

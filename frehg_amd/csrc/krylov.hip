@@ -1245,7 +1245,10 @@ void Krylov::build() {
   FREHG_HIP(hipStreamSynchronize(s_));
 }
 
-Krylov::~Krylov() { release(); }
+Krylov::~Krylov() {
+  resident_leave();
+  release();
+}
 
 void Krylov::release() {
   if (borrowed_) return;  // the workspace belongs to the caller
@@ -1482,9 +1485,14 @@ int Krylov::cg_outcome(double* res_norm, double* rhs_norm, bool* converged) {
 
 namespace {
 // Launches of the resident solver with more than one block wait for one another's blocks, so two of
-// them (on two contexts' streams) must not share a device: each holds its device's lock until it is done.
+// them (on two contexts' streams) must not share a device. Per device: the stream of the last such launch;
+// a launch on another stream first waits until that one has drained.
 constexpr int kMaxDevices = 64;
-std::mutex g_resident_mu[kMaxDevices];
+struct ResidentTurn {
+  std::mutex mu;
+  hipStream_t last = nullptr;
+  const void* owner = nullptr;
+} g_resident[kMaxDevices];
 
 template <typename T, bool THREE_D>
 void launch_resident(int cpt, unsigned int nblk, size_t lds, hipStream_t s, const CgResidentArgs<T>& a) {
@@ -1499,11 +1507,10 @@ void launch_resident(int cpt, unsigned int nblk, size_t lds, hipStream_t s, cons
 }  // namespace
 
 template <typename T>
-bool Krylov::cg_resident(const StencilView<T>& A, const T* b, const T* bn, T* x, const unsigned char* fixed, bool zero,
-                         bool guard, double rtol, double atol, int max_it, const T* r0, const KrylovCtl* started) {
+void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T* x, const unsigned char* fixed,
+                             bool zero, bool guard, double rtol, double atol, int max_it, const T* r0,
+                             const KrylovCtl* started) {
   const ResidentPlan& pl = plan_[sizeof(T) == 4 ? 1 : 0];
-  std::unique_lock<std::mutex> lock;
-  if (pl.nblk > 1) lock = std::unique_lock<std::mutex>(g_resident_mu[device_ % kMaxDevices]);
   if (++launch_ >= (1u << 20)) {  // the tags start again: no old one may be left
     launch_ = 1;
     if (mail_words_) clear_exchange();
@@ -1517,7 +1524,7 @@ bool Krylov::cg_resident(const StencilView<T>& A, const T* b, const T* bn, T* x,
   a.fixed = fixed;
   a.r0 = r0;
   a.ctl = started;
-  // the outcome goes straight to pinned host memory (a borrowed workspace has none: copied below)
+  // the outcome goes straight to pinned host memory (a borrowed workspace has none: resident_wait copies it)
   KrylovCtl* out = borrowed_ ? ctl_ : host_ctl_;
   host_ctl_[1].iters = 0;
   a.out = out;
@@ -1539,13 +1546,63 @@ bool Krylov::cg_resident(const StencilView<T>& A, const T* b, const T* bn, T* x,
   }
   a.mail = mail_;
   a.launch = launch_;
+  std::unique_lock<std::mutex> lock;
+  if (pl.nblk > 1) {
+    ResidentTurn& turn = g_resident[device_ % kMaxDevices];
+    lock = std::unique_lock<std::mutex>(turn.mu);
+    if (turn.last && turn.last != s_) FREHG_HIP(hipStreamSynchronize(turn.last));
+    turn.last = s_;
+    turn.owner = this;
+  }
   if (three_d_) launch_resident<T, true>(pl.cpt, pl.nblk, pl.lds, s_, a);
   else launch_resident<T, false>(pl.cpt, pl.nblk, pl.lds, s_, a);
-  if (borrowed_) FREHG_HIP(hipMemcpyAsync(host_ctl_, ctl_, 2 * sizeof(KrylovCtl), hipMemcpyDeviceToHost, s_));
-  FREHG_HIP(hipStreamSynchronize(s_));
+}
+
+bool Krylov::resident_ended() {
   if (host_ctl_[1].iters == 0) return true;
   plan_[0] = plan_[1] = ResidentPlan{};
   return false;
+}
+
+void Krylov::resident_leave() {
+  ResidentTurn& turn = g_resident[device_ % kMaxDevices];
+  std::lock_guard<std::mutex> lock(turn.mu);
+  if (turn.owner != this) return;
+  (void)hipStreamSynchronize(s_);
+  turn.last = nullptr;
+  turn.owner = nullptr;
+}
+
+template <typename T>
+bool Krylov::cg_resident(const StencilView<T>& A, const T* b, const T* bn, T* x, const unsigned char* fixed, bool zero,
+                         bool guard, double rtol, double atol, int max_it, const T* r0, const KrylovCtl* started) {
+  resident_launch<T>(A, b, bn, x, fixed, zero, guard, rtol, atol, max_it, r0, started);
+  if (borrowed_) FREHG_HIP(hipMemcpyAsync(host_ctl_, ctl_, 2 * sizeof(KrylovCtl), hipMemcpyDeviceToHost, s_));
+  FREHG_HIP(hipStreamSynchronize(s_));
+  return resident_ended();
+}
+
+bool Krylov::enqueue(const StencilView<double>& A, const double* b, const double* bn, double* x,
+                     const unsigned char* fixed, bool x0_zero, const KrylovConfig& cfg) {
+  if (cfg.ksp != FREHG_KSP_CG || cfg.precision != 0 || borrowed_ || !resident(0) || !A.symmetric()) return false;
+  resident_launch<double>(A, b, bn, x, fixed, x0_zero, false, cfg.rtol, cfg.atol, cfg.max_it, nullptr, nullptr);
+  return true;
+}
+
+bool Krylov::finish_queued(SolveResult* res) {
+  if (!resident_ended()) return false;
+  bool conv = false;
+  *res = SolveResult{};
+  res->iterations = cg_outcome<double>(&res->residual_norm, &res->rhs_norm, &conv);
+  res->converged = conv;
+  if (!conv) throw_not_converged(*res);
+  return true;
+}
+
+void Krylov::throw_not_converged(const SolveResult& res) const {
+  throw ConvergenceError(std::string("Krylov ") + (three_d_ ? "3D" : "2D") + ": not converged within max_it (" +
+                         std::to_string(res.iterations) + " iterations, ||D^-1 r|| = " +
+                         std::to_string(res.residual_norm) + ", ||D^-1 b|| = " + std::to_string(res.rhs_norm) + ")");
 }
 
 template <typename T>
@@ -1724,10 +1781,7 @@ SolveResult Krylov::solve(const StencilView<double>& A, const StencilView<float>
                                  three_d_ ? FREHG_KT_GW_SPMV : FREHG_KT_SW_SPMV);
     res.guess_rejected = rej;
     res.converged = conv;
-    if (!conv)
-      throw ConvergenceError(std::string("Krylov ") + (three_d_ ? "3D" : "2D") + ": not converged within max_it (" +
-                             std::to_string(res.iterations) + " iterations, ||D^-1 r|| = " +
-                             std::to_string(res.residual_norm) + ", ||D^-1 b|| = " + std::to_string(res.rhs_norm) + ")");
+    if (!conv) throw_not_converged(res);
     return res;
   }
   // FP32 inner / FP64 outer iterative refinement.

@@ -122,6 +122,14 @@ class Krylov {
   };
   SweepTarget first_sweep_target();
 
+  // solve() without the wait, where the solve is one launch (FP64 CG on a resident-size operator): queues
+  // it and returns true, or returns false and does nothing. After the stream has drained, finish_queued gives
+  // the outcome as solve() would (it throws as solve() does), or false when the solve has to be done again
+  // with solve() (x holds a mixture of iterates) together with the work queued behind it.
+  bool enqueue(const StencilView<double>& A, const double* b, const double* bn, double* x, const unsigned char* fixed,
+               bool x0_zero, const KrylovConfig& cfg);
+  bool finish_queued(SolveResult* res);
+
   // CG SpMV launch shape per precision (0 FP64, 1 FP32): cells per lane (1: one column per
   // thread on 64 x 4 tiles; 2: two adjacent columns per lane on 128 x 4 tiles, paired aligned
   // loads, x-neighbours by wave shifts) and layers per block of the z-march (kc).
@@ -152,12 +160,19 @@ class Krylov {
  private:
   void setup_resident();
   void clear_exchange();
-  // Solves by one launch of the resident kernel and waits for it; the outcome is in host_ctl_. False when a
-  // wait inside the launch ran out (x may hold a mixture of iterates; the instance then streams).
-  // r0 / started: a solve begun by a refinement sweep (x0 = 0).
+  // One launch of the resident kernel (r0 / started: a solve begun by a refinement sweep, x0 = 0); once the
+  // stream has drained its outcome is in host_ctl_ and resident_ended() is false when a wait inside the
+  // launch ran out (x may hold a mixture of iterates; the instance then streams).
+  template <typename T>
+  void resident_launch(const StencilView<T>& A, const T* b, const T* bn, T* x, const unsigned char* fixed, bool zero,
+                       bool guard, double rtol, double atol, int max_it, const T* r0, const KrylovCtl* started);
+  bool resident_ended();
+  void resident_leave();
+  // The launch, and the wait for it.
   template <typename T>
   bool cg_resident(const StencilView<T>& A, const T* b, const T* bn, T* x, const unsigned char* fixed, bool zero,
                    bool guard, double rtol, double atol, int max_it, const T* r0, const KrylovCtl* started);
+  [[noreturn]] void throw_not_converged(const SolveResult& res) const;
   // Errors, counters and norms of a finished CG solve from host_ctl_.
   template <typename T>
   int cg_outcome(double* res_norm, double* rhs_norm, bool* converged);

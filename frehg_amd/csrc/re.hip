@@ -139,7 +139,8 @@ __global__ __launch_bounds__(NT) void k_re_realloc_iter(K P, FA fa, const unsign
 // Reallocation + clamp + moisture BCs; ledger partials (sum theta^{n+1} V, sum (theta^{n+1} -
 // theta_c) V) to part[3..4][nblocks] and max |h^{n+1} - h^n| to mx[nblocks].
 template <class K, int ZF, class FA>
-__global__ __launch_bounds__(NT) void k_re_finalize(K P, FA fa, const unsigned char* __restrict__ sat0,
+__global__ __launch_bounds__(NT) void k_re_finalize(K P, FA fa, const int* __restrict__ changed,
+                                                     const unsigned char* __restrict__ sat0,
                                                      const unsigned char* __restrict__ fin,
                                                      const double* __restrict__ wch, const double* __restrict__ hwc,
                                                      const double* __restrict__ hn, double* __restrict__ wc,
@@ -149,6 +150,7 @@ __global__ __launch_bounds__(NT) void k_re_finalize(K P, FA fa, const unsigned c
                                                      unsigned int nblocks) {
   __shared__ double lds[NT / kWave];
   __shared__ double lmax[NT / kWave];
+  if (changed && *changed) return;  // the sweep before changed the saturation state: not its fixed point yet
   TileId b;
   const Cell t = tile_cell<ZF>(P.g, b);
   double l_after = 0.0, l_adj = 0.0, dh = 0.0;
@@ -165,6 +167,56 @@ __global__ __launch_bounds__(NT) void k_re_finalize(K P, FA fa, const unsigned c
     part[4 * nblocks + b.linear] = bs;
     mx[b.linear] = m;
     mx[nblocks + b.linear] = 0.0;
+  }
+}
+
+// The step's results from its block partials, to (pinned host) out[0..5]: five ledger sums (rows of n in
+// part) and the maximum of mx[0..n); out[7] = *flag. One block: one launch of about 3 us where five sums and
+// a maximum in two stages each took four; longer rows (more than kResultsOne) are first brought to kRedStage
+// entries per row by k_re_results_stage.
+constexpr unsigned int kResultsOne = 4096;
+constexpr int kResultsNT = 512;
+
+__device__ inline void results_of(const double* part, const double* mx, unsigned int n, unsigned int lo, unsigned int hi,
+                                  double (&v)[5], double* m) {
+  double a = 0.0;
+  for (unsigned int i = lo + threadIdx.x; i < hi; i += kResultsNT) {
+#pragma unroll
+    for (int q = 0; q < 5; ++q) v[q] += part[(size_t)q * n + i];
+    a = fmax(a, mx[i]);
+  }
+  __shared__ double lds[5 * (kResultsNT / kWave)];
+  __shared__ double lmax[kResultsNT / kWave];
+  a = wave_max(a);
+  if ((threadIdx.x & (kWave - 1)) == 0) lmax[threadIdx.x / kWave] = a;
+  block_sums<kResultsNT, 5>(v, lds);  // (its barriers order lmax too)
+  double r = lmax[0];
+  for (int q = 1; q < kResultsNT / kWave; ++q) r = fmax(r, lmax[q]);
+  *m = r;
+}
+
+__global__ __launch_bounds__(kResultsNT) void k_re_results_stage(const double* part, const double* mx, unsigned int n,
+                                                                 double* out) {
+  const unsigned int chunk = (n + gridDim.x - 1) / gridDim.x;
+  const unsigned int lo = blockIdx.x * chunk, hi = min(n, lo + chunk);
+  double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, m;
+  results_of(part, mx, n, lo, hi, v, &m);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < 5; ++q) out[q * gridDim.x + blockIdx.x] = v[q];
+    out[5 * gridDim.x + blockIdx.x] = m;
+  }
+}
+
+__global__ __launch_bounds__(kResultsNT) void k_re_results(const double* part, const double* mx, unsigned int n,
+                                                           const int* flag, double* out) {
+  double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, m;
+  results_of(part, mx, n, 0, n, v, &m);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < 5; ++q) out[q] = v[q];
+    out[5] = m;
+    out[7] = flag ? (double)*flag : 0.0;
   }
 }
 
@@ -500,7 +552,7 @@ void ReState::build(const frehg_re_params& p) {
   FREHG_HIP(hipMalloc(&red_, 2 * (size_t)nb * sizeof(double)));
   FREHG_HIP(hipMalloc(&led_, 7 * (size_t)nb * sizeof(double)));
   FREHG_HIP(hipMalloc(&dres_, 16 * sizeof(double)));
-  FREHG_HIP(hipMalloc(&red2_, 5 * kRedStage * sizeof(double)));
+  FREHG_HIP(hipMalloc(&red2_, 6 * kRedStage * sizeof(double)));
   FREHG_HIP(hipHostMalloc(&hres_, 16 * sizeof(double), hipHostMallocDefault));
   FREHG_HIP(hipMalloc(&dcount_, 16));
   FREHG_HIP(hipMemsetAsync(dcount_, 0, 16, s_));
@@ -897,7 +949,11 @@ void ReState::step(frehg_re_stats* st) {
   }
   StencilView<double> A{D_, ax_, ay_, az_};
   StencilView<float> A32{D32_, ax32_, ay32_, az32_};
-  SolveResult sr = kry_->solve(A, mixed ? &A32 : nullptr, rhs_, nullptr, h_, nullptr, x0_zero, guard, kc, swept);
+  // An FP64 solve that is one launch is queued and its outcome read with the next results the host waits for
+  // (the Picard test, or the end of the step).
+  SolveResult sr;
+  bool queued = !mixed && !guard && !logging && kry_->enqueue(A, rhs_, nullptr, h_, nullptr, x0_zero, kc);
+  if (!queued) sr = kry_->solve(A, mixed ? &A32 : nullptr, rhs_, nullptr, h_, nullptr, x0_zero, guard, kc, swept);
   // A learned Picard start whose residual did not drop below the zero guess's: the solve above
   // started from zero, but on the operator assembled at the rejected head. The loop restarts as
   // the plain method: h^0 = h^n, K and C at h^n, x0 = 0.
@@ -921,16 +977,33 @@ void ReState::step(frehg_re_stats* st) {
     sr.fallback_fp64 = sr.fallback_fp64 || s0.fallback_fp64;
     from_hn = true;
   }
-  local.solve.iterations = sr.iterations;
-  local.solve.refinements = sr.refinements;
-  local.solve.residual_norm = sr.residual_norm;
-  local.solve.rhs_norm = sr.rhs_norm;
-  local.solve.converged = sr.converged ? 1 : 0;
-  local.solve.fallback = sr.fallback_fp64 ? 1 : 0;
+  bool refined = sr.refinements > 0;  // the last solve took a refinement (mixed precision)
+  bool unchanged = false;             // the last solve returned its start unchanged
+  auto book = [&](const SolveResult& r, bool first) {  // a solve's outcome into the step's
+    local.solve.iterations += r.iterations;
+    local.solve.refinements += r.refinements;
+    local.solve.residual_norm = r.residual_norm;
+    local.solve.rhs_norm = r.rhs_norm;
+    local.solve.converged = ((first || local.solve.converged) && r.converged) ? 1 : 0;
+    local.solve.fallback |= r.fallback_fp64 ? 1 : 0;
+    refined = r.refinements > 0;
+    unchanged = r.iterations == 0 && r.refinements == 0 && !r.fallback_fp64;
+  };
+  if (!queued) book(sr, true);
   local.guess_fallback = sr.guess_rejected ? 1 : 0;
   local.picard_iterations = 1;
   local.picard_converged = p_.picard_max > 1 ? 0 : 1;
-  bool refined = sr.refinements > 0;  // the last solve took a refinement (mixed precision)
+  // Once the stream has drained: the outcome of a queued solve. When it has to be solved again (true), the
+  // work queued behind it has to be queued again too.
+  auto resolve = [&](bool zero, bool first) -> bool {
+    if (!queued) return false;
+    queued = false;
+    SolveResult r;
+    const bool again = !kry_->finish_queued(&r);
+    if (again) r = kry_->solve(A, nullptr, rhs_, nullptr, h_, nullptr, zero, false, kc);
+    book(r, first);
+    return again;
+  };
   // Picard outer loop (picard_max > 1; a new method, the reference's step is its first iterate):
   // K and C at the iterate h^m with its head-BC ghosts, the storage and rhs terms at time level n
   // as in the predictor, solve for h^{m+1} (from x0 = 0 with the zero guess, else from h^m); stop
@@ -940,15 +1013,15 @@ void ReState::step(frehg_re_stats* st) {
   bool post_done = false, flux_done = false;
   for (int m = 1; p_.picard_max > 1; ++m) {
     const double* ref = (m == 1 && from_hn) ? hn_ : hp_;
+    const bool zero = p_.initial_guess == FREHG_GUESS_ZERO;
     with_soil_variant(P, [&](const auto& PK) {
       using K = std::decay_t<decltype(PK)>;
       hipLaunchKernelGGL((k_re_post_delta<K, 1>), grid, blk, 0, s_, PK, h_, kr_, ch_, wch_, ref, hp_, red_, nbl);
       FREHG_LAUNCH_CHECK();
     });
     post_done = true;
-    reduce_maxmin(red_, nbl, red2_, dres_, s_);
+    reduce_maxmin(red_, nbl, red2_, hres_, s_);
     FREHG_LAUNCH_CHECK();
-    const bool zero = p_.initial_guess == FREHG_GUESS_ZERO;
     // A solve from h^m first tests the residual of h^m on the system assembled at h^m and returns
     // h^m unchanged when the test passes, which ends the loop (below). That test is taken here
     // on rows formed in registers, without storing the system; only when it fails is the system
@@ -979,20 +1052,36 @@ void ReState::step(frehg_re_stats* st) {
                              (const double*)wcn_, (const double*)hn_, (const double*)h_, red_, nbl);
         FREHG_LAUNCH_CHECK();
       });
-      reduce_sums(red_, nbl, 2, red2_, dres_ + 11, s_);
+      reduce_sums(red_, nbl, 2, red2_, hres_ + 11, s_);
       FREHG_LAUNCH_CHECK();
     }
-    // [0] the Picard test's max |dh|, [11..12] the residual test's sums (the slots between are
-    // rewritten by the ledger copy at the end of the step)
-    FREHG_HIP(hipMemcpyAsync(hres_, dres_, (spec ? 13 : 1) * sizeof(double), hipMemcpyDeviceToHost, s_));
+    // hres_ (written by the reductions): [0] the Picard test's max |dh|, [11..12] the residual test's sums
     FREHG_HIP(hipStreamSynchronize(s_));
-    if (hres_[0] <= p_.picard_tol) {
+    // (a solve that had to be done again invalidates what was queued behind it: the loop goes on)
+    const bool again = resolve(m == 1 ? x0_zero : zero, m == 1);
+    if (again) {
+      with_soil_variant(P, [&](const auto& PK) {
+        using K = std::decay_t<decltype(PK)>;
+        hipLaunchKernelGGL((k_re_post_delta<K, 1>), grid, blk, 0, s_, PK, h_, kr_, ch_, wch_, (const double*)hp_,
+                           hp_, red_, nbl);
+        FREHG_LAUNCH_CHECK();
+      });
+    }
+    if (m > 1 && !zero && unchanged && !again) {
+      // a solve from h^{m-1} that returned it unchanged ended the loop before this iterate in the waiting form;
+      // here the passes at h^m = h^{m-1} have repeated their results
+      local.picard_converged = 1;
+      flux_done = spec && check_flux_;
+      skip_check_ &= ~(m - 1 < 32 ? 1u << (m - 1) : 0u);
+      break;
+    }
+    if (!again && hres_[0] <= p_.picard_tol) {
       local.picard_converged = 1;
       flux_done = spec && check_flux_;
       break;
     }
     if (m >= p_.picard_max) break;  // the cap: the step continues from the last iterate
-    if (spec) {
+    if (spec && !again) {
       const double rr = hres_[11], bb = hres_[12];
       const double ttol = std::fmax(kc.rtol * std::sqrt(bb), kc.atol);
       if (rr <= ttol * ttol) {
@@ -1014,19 +1103,14 @@ void ReState::step(frehg_re_stats* st) {
     const bool fresh32 = mixed && (zero || refined);
     const unsigned int swept_m = assemble(fresh32, !zero);
     post_done = false;
-    const SolveResult sm = kry_->solve(A, mixed ? &A32 : nullptr, rhs_, nullptr, h_, nullptr, zero, false, kc, swept_m);
-    local.solve.iterations += sm.iterations;
-    local.solve.refinements += sm.refinements;
-    local.solve.residual_norm = sm.residual_norm;
-    local.solve.rhs_norm = sm.rhs_norm;
-    local.solve.converged = (local.solve.converged && sm.converged) ? 1 : 0;
-    local.solve.fallback |= sm.fallback_fp64 ? 1 : 0;
     local.picard_iterations = m + 1;
-    refined = sm.refinements > 0;
+    queued = !mixed && !logging && kry_->enqueue(A, rhs_, nullptr, h_, nullptr, zero, kc);
+    if (queued) continue;
+    book(kry_->solve(A, mixed ? &A32 : nullptr, rhs_, nullptr, h_, nullptr, zero, false, kc, swept_m), false);
     // A solve from h^m that returned it unchanged (converged at its first residual check, no
     // update): h^{m+1} = h^m bit for bit, so the test passes (max |dh| = 0), and the post-solve
     // pass at h^{m+1} would repeat the one just done at h^m, whose results are still in place.
-    if (!zero && sm.iterations == 0 && sm.refinements == 0 && !sm.fallback_fp64) {
+    if (!zero && unchanged) {
       post_done = true;
       local.picard_converged = 1;
       skip_check_ &= ~bit;
@@ -1034,83 +1118,116 @@ void ReState::step(frehg_re_stats* st) {
     }
   }
   if (logging && inc0) mlp_->log_pair(*this, hn_, h_, depth_, inc0);
-  // Without lazy fluxes finalize writes the final head over the post-solve head: keep the latter
-  // in hp_ for the next step's increment.
-  if (track_inc && !lazy_flux_) {
-    hipLaunchKernelGGL(k_copy_interior, grid, blk, 0, s_, g_, (const double*)h_, hp_);
-    FREHG_LAUNCH_CHECK();
-  }
-  if (!flux_done) {
-    hipEvent_t ev0 = prof_->start(FREHG_KT_GW_CORRECT);
-    hipEvent_t ev1 = prof_->stop();
-    with_soil_variant(P, [&](const auto& PK) {
-      using K = std::decay_t<decltype(PK)>;
-      if (!post_done) {
-        hipExtLaunchKernelGGL((k_re_post<K, 1>), grid, blk, 0, s_, ev0, nullptr, 0, PK, h_, kr_, ch_, wch_);
-        FREHG_LAUNCH_CHECK();
-      }
-      hipExtLaunchKernelGGL((k_re_flux_correct<K, 1>), grid, blk, 0, s_, post_done ? ev0 : nullptr, ev1, 0, PK,
-                            (const double*)h_,
-                            (const double*)kr_, (const double*)hn_, (const double*)wcn_, (const double*)wch_, Kx_, Ky_,
-                            Kz_, qx_, qy_, qz_, wc_, hwc_, sat0_, cand_, lazy_flux_ ? kf_ : nullptr, led_, nbl,
-                            dflag_, kSweepFlags);
+  // The step's results (see k_re_results) to hres_ + 2.
+  auto results = [&](const int* flag) {
+    const double* mx = led_ + 5 * (size_t)nbl;
+    if (nbl > kResultsOne) {
+      hipLaunchKernelGGL(k_re_results_stage, dim3(kRedStage), dim3(kResultsNT), 0, s_, (const double*)led_, mx, nbl,
+                         red2_);
       FREHG_LAUNCH_CHECK();
-    });
-  }
-  // Reallocation fixed point: sweep until the saturation state stops changing. Sweep 0 reads
-  // sat0 itself; later sweeps alternate between satA and satB. Sweep s reports a change in
-  // dflag_[s] (cleared by the flux kernel above).
+      hipLaunchKernelGGL(k_re_results, dim3(1), dim3(kResultsNT), 0, s_, (const double*)red2_,
+                         (const double*)red2_ + 5 * kRedStage, kRedStage, flag, hres_ + 2);
+    } else {
+      hipLaunchKernelGGL(k_re_results, dim3(1), dim3(kResultsNT), 0, s_, (const double*)led_, mx, nbl, flag,
+                         hres_ + 2);
+    }
+    FREHG_LAUNCH_CHECK();
+  };
+  // Sweep `it` of the reallocation fixed point. Sweep 0 reads sat0 itself; later sweeps alternate between satA
+  // and satB. Sweep s reports a change in dflag_[s] (cleared by the flux kernel).
   const unsigned char* prev = sat0_;
-  for (int it = 0; it < g_.nx * g_.ny * g_.nz + 1; ++it) {
+  auto sweep_flag = [&](int it) { return dflag_ + (it < kSweepFlags ? it : kSweepFlags - 1); };
+  auto realloc_sweep = [&](int it) {
     unsigned char* next = (it & 1) ? satB_ : satA_;
-    const int f = it < kSweepFlags ? it : kSweepFlags - 1;
-    if (it >= kSweepFlags) FREHG_HIP(hipMemsetAsync(dflag_ + f, 0, sizeof(int), s_));
+    int* flag = sweep_flag(it);
+    if (it >= kSweepFlags) FREHG_HIP(hipMemsetAsync(flag, 0, sizeof(int), s_));
     with_soil_variant(P, [&](const auto& PK) {
       using K = std::decay_t<decltype(PK)>;
       if (lazy_flux_)
         hipLaunchKernelGGL((k_re_realloc_iter<K, FacesF>), grid, blk, 0, s_, PK, FacesF{kf_},
-                           (const unsigned char*)sat0_, (const unsigned char*)cand_, prev, next, dflag_ + f);
+                           (const unsigned char*)sat0_, (const unsigned char*)cand_, prev, next, flag);
       else
         hipLaunchKernelGGL((k_re_realloc_iter<K, FacesK>), grid, blk, 0, s_, PK, FacesK{Kx_, Ky_},
-                           (const unsigned char*)sat0_, (const unsigned char*)cand_, prev, next, dflag_ + f);
+                           (const unsigned char*)sat0_, (const unsigned char*)cand_, prev, next, flag);
       FREHG_LAUNCH_CHECK();
     });
-    FREHG_HIP(hipMemcpyAsync(hflag_, dflag_ + f, sizeof(int), hipMemcpyDeviceToHost, s_));
-    FREHG_HIP(hipStreamSynchronize(s_));
     prev = next;
-    if (hflag_[0] == 0) break;
+  };
+  // Reallocation branches, clamp, ghosts and ledger, unless *changed. Lazy fluxes: the final head goes to hp_
+  // and h_ keeps the post-solve head; the swap below leaves the final head in h_ and the post-solve head (a
+  // flux rebuild input) in hp_.
+  auto finalize = [&](const int* changed) {
+    with_soil_variant(P, [&](const auto& PK) {
+      using K = std::decay_t<decltype(PK)>;
+      if (lazy_flux_)
+        hipLaunchKernelGGL((k_re_finalize<K, 0, FacesF>), grid, blk, 0, s_, PK, FacesF{kf_}, changed,
+                           (const unsigned char*)sat0_, prev, (const double*)wch_, (const double*)hwc_,
+                           (const double*)hn_, wc_, h_, hp_, hmod_, led_, led_ + 5 * (size_t)nbl, nbl);
+      else
+        hipLaunchKernelGGL((k_re_finalize<K, 0, FacesK>), grid, blk, 0, s_, PK, FacesK{Kx_, Ky_}, changed,
+                           (const unsigned char*)sat0_, prev, (const double*)wch_, (const double*)hwc_,
+                           (const double*)hn_, wc_, h_, nullptr, hmod_, led_, led_ + 5 * (size_t)nbl, nbl);
+      FREHG_LAUNCH_CHECK();
+    });
+  };
+  // From the fluxes to the results of the first reallocation sweep, queued without a wait: the finalize kernel
+  // does nothing when that sweep changed the saturation state (few steps do), and the host then continues the
+  // fixed point below.
+  auto tail = [&] {
+    // Without lazy fluxes finalize writes the final head over the post-solve head: keep the latter
+    // in hp_ for the next step's increment.
+    if (track_inc && !lazy_flux_) {
+      hipLaunchKernelGGL(k_copy_interior, grid, blk, 0, s_, g_, (const double*)h_, hp_);
+      FREHG_LAUNCH_CHECK();
+    }
+    if (!flux_done) {
+      hipEvent_t ev0 = prof_->start(FREHG_KT_GW_CORRECT);
+      hipEvent_t ev1 = prof_->stop();
+      with_soil_variant(P, [&](const auto& PK) {
+        using K = std::decay_t<decltype(PK)>;
+        if (!post_done) {
+          hipExtLaunchKernelGGL((k_re_post<K, 1>), grid, blk, 0, s_, ev0, nullptr, 0, PK, h_, kr_, ch_, wch_);
+          FREHG_LAUNCH_CHECK();
+        }
+        hipExtLaunchKernelGGL((k_re_flux_correct<K, 1>), grid, blk, 0, s_, post_done ? ev0 : nullptr, ev1, 0, PK,
+                              (const double*)h_, (const double*)kr_, (const double*)hn_, (const double*)wcn_,
+                              (const double*)wch_, Kx_, Ky_, Kz_, qx_, qy_, qz_, wc_, hwc_, sat0_, cand_,
+                              lazy_flux_ ? kf_ : nullptr, led_, nbl, dflag_, kSweepFlags);
+        FREHG_LAUNCH_CHECK();
+      });
+    }
+    prev = sat0_;
+    realloc_sweep(0);
+    finalize(sweep_flag(0));
+    results(sweep_flag(0));
+    if (p_.initial_guess == FREHG_GUESS_LEARNED)
+      FREHG_HIP(hipMemcpyAsync(hres_ + 10, dres_ + 10, sizeof(double), hipMemcpyDeviceToHost, s_));
+    FREHG_HIP(hipStreamSynchronize(s_));
+  };
+  tail();
+  if (resolve(x0_zero, true)) tail();  // (the predictor's queued solve)
+  if (hres_[9] != 0.0) {
+    for (int it = 1; it < g_.nx * g_.ny * g_.nz + 1; ++it) {
+      realloc_sweep(it);
+      FREHG_HIP(hipMemcpyAsync(hflag_, sweep_flag(it), sizeof(int), hipMemcpyDeviceToHost, s_));
+      FREHG_HIP(hipStreamSynchronize(s_));
+      if (hflag_[0] == 0) break;
+    }
+    finalize(nullptr);
+    results(nullptr);
+    FREHG_HIP(hipStreamSynchronize(s_));
   }
-  // Lazy fluxes: the final head goes to hp_ and h_ keeps the post-solve head; the swap below
-  // leaves the final head in h_ and the post-solve head (a flux rebuild input) in hp_.
-  with_soil_variant(P, [&](const auto& PK) {
-    using K = std::decay_t<decltype(PK)>;
-    if (lazy_flux_)
-      hipLaunchKernelGGL((k_re_finalize<K, 0, FacesF>), grid, blk, 0, s_, PK, FacesF{kf_},
-                         (const unsigned char*)sat0_, prev, (const double*)wch_, (const double*)hwc_,
-                         (const double*)hn_, wc_, h_, hp_, hmod_, led_, led_ + 5 * (size_t)nbl, nbl);
-    else
-      hipLaunchKernelGGL((k_re_finalize<K, 0, FacesK>), grid, blk, 0, s_, PK, FacesK{Kx_, Ky_},
-                         (const unsigned char*)sat0_, prev, (const double*)wch_, (const double*)hwc_,
-                         (const double*)hn_, wc_, h_, nullptr, hmod_, led_, led_ + 5 * (size_t)nbl, nbl);
-    FREHG_LAUNCH_CHECK();
-  });
   if (lazy_flux_) {
     std::swap(h_, hp_);
     flux_pending_ = true;
   }
-  // ledger: [before, storage_ss, boundary_in, after, adjust] sums, then max |dh|
-  reduce_sums(led_, nbl, 5, red2_, dres_ + 2, s_);
-  FREHG_LAUNCH_CHECK();
-  reduce_maxmin(led_ + 5 * (size_t)nbl, nbl, red2_, dres_ + 7, s_);
-  FREHG_LAUNCH_CHECK();
   if (p_.adaptive_dt) {
     materialize_fluxes();
     const unsigned int nb = grid.x * grid.y * grid.z;
     hipLaunchKernelGGL(k_re_dtadapt, grid, blk, 0, s_, P, qx_, qy_, qz_, wc_, red_, nb);
     FREHG_LAUNCH_CHECK();
-    reduce_maxmin(red_, nb, red2_, dres_, s_);
+    reduce_maxmin(red_, nb, red2_, hres_, s_);
     FREHG_LAUNCH_CHECK();
-    FREHG_HIP(hipMemcpyAsync(hres_, dres_, 2 * sizeof(double), hipMemcpyDeviceToHost, s_));
     FREHG_HIP(hipStreamSynchronize(s_));
     // ReSolver::adaptiveTimeStep (ReSolver.cpp:890-928)
     const double dq_max = hres_[0], dt_Comin = hres_[1];
@@ -1122,8 +1239,6 @@ void ReState::step(frehg_re_stats* st) {
     if (p_.dt < p_.dt_min) p_.dt = p_.dt_min;
     dtn_ = p_.dt;
   }
-  FREHG_HIP(hipMemcpyAsync(hres_ + 2, dres_ + 2, 9 * sizeof(double), hipMemcpyDeviceToHost, s_));
-  FREHG_HIP(hipStreamSynchronize(s_));
   // a network output that was not finite: those cells started from h^n + d^{n-1} instead
   if (p_.initial_guess == FREHG_GUESS_LEARNED && hres_[10] != 0.0) local.guess_fallback = 1;
   local.mass_before = hres_[2];
