@@ -57,6 +57,7 @@ struct CgResidentArgs {
   const KrylovCtl* ctl;      // and its control block
   KrylovCtl* out;            // result (device or pinned host memory)
   int* timeout;              // set to 1 when a wait ends without its word
+  int* failed;               // device word for kernels queued behind: set to 1 unless the solve converges
   double rtol, atol;
   int max_it, guard, x0_zero;
   int tx, ty, tz, ntx, nty, ntz;  // cells per tile, tiles
@@ -70,6 +71,9 @@ __device__ __forceinline__ void cg_put(unsigned long long* p, unsigned long long
 }
 __device__ __forceinline__ unsigned long long cg_get(const unsigned long long* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void cg_fail(int* failed) {
+  __hip_atomic_store(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ unsigned long long cg_tagged(unsigned int tag, unsigned int v) {
   return ((unsigned long long)tag << 32) | v;
@@ -372,7 +376,10 @@ __global__ __launch_bounds__(kCgNT) void k_cg_resident(CgResidentArgs<T> P) {
     }
     cg_block_sums<N>(v, red, flip++);  // its barrier also makes `dead` visible
     if (dead) {
-      if (tid == 0) __hip_atomic_store(P.timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      if (tid == 0) {
+        __hip_atomic_store(P.timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        cg_fail(P.failed);
+      }
       return false;
     }
     return true;
@@ -477,6 +484,7 @@ __global__ __launch_bounds__(kCgNT) void k_cg_resident(CgResidentArgs<T> P) {
     o.max_it = P.max_it;
     o.guess_rejected = rejected;
     *P.out = o;
+    if (!conv) cg_fail(P.failed);
   }
 }
 

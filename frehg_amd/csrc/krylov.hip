@@ -1299,6 +1299,7 @@ void Krylov::autotune(const StencilView<T>& A) {
   if (!three_d_) return;
   if (prec == 1) ensure_mixed();
   KrylovCtl* tctl = ctl_ + 2;
+  failed_dirty_ = true;  // (the same word)
   FREHG_HIP(hipMemsetAsync(tctl, 0, sizeof(KrylovCtl), s_));
   T* p0 = prec ? (T*)p032_ : (T*)p0_;
   T* p1 = prec ? (T*)p132_ : (T*)p1_;
@@ -1529,6 +1530,9 @@ void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T
   host_ctl_[1].iters = 0;
   a.out = out;
   a.timeout = &out[1].iters;
+  a.failed = failed_flag();
+  if (failed_dirty_) FREHG_HIP(hipMemsetAsync(a.failed, 0, sizeof(int), s_));
+  failed_dirty_ = true;  // until its outcome has been seen
   a.rtol = rtol;
   a.atol = atol;
   a.max_it = max_it;
@@ -1559,7 +1563,10 @@ void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T
 }
 
 bool Krylov::resident_ended() {
-  if (host_ctl_[1].iters == 0) return true;
+  if (host_ctl_[1].iters == 0) {
+    failed_dirty_ = !host_ctl_->converged;
+    return true;
+  }
   plan_[0] = plan_[1] = ResidentPlan{};
   return false;
 }

@@ -129,6 +129,8 @@ class Krylov {
   bool enqueue(const StencilView<double>& A, const double* b, const double* bn, double* x, const unsigned char* fixed,
                bool x0_zero, const KrylovConfig& cfg);
   bool finish_queued(SolveResult* res);
+  // Device word that a queued solve sets to 1 unless it converges, for the kernels queued behind it.
+  int* failed_flag() const { return &ctl_[2].iters; }
 
   // CG SpMV launch shape per precision (0 FP64, 1 FP32): cells per lane (1: one column per
   // thread on 64 x 4 tiles; 2: two adjacent columns per lane on 128 x 4 tiles, paired aligned
@@ -242,6 +244,7 @@ class Krylov {
   KrylovCtl host_ctl_own_[2] = {};  // host mirrors of the control blocks in borrowed mode
   ResidentPlan plan_[2];          // resident CG solve per precision (0 FP64, 1 FP32)
   int device_ = 0;
+  bool failed_dirty_ = true;      // failed_flag() may hold a failure
   unsigned int launch_ = 0;       // resident launches of this instance (the tag of their exchanges)
   unsigned long long *halo_[4] = {}, *mail_ = nullptr;  // its exchange buffers: low, low, high, high words; sums
   size_t mail_words_ = 0;

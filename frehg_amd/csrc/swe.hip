@@ -1,22 +1,23 @@
 // Semi-implicit shallow-water step on the GPU, following SweSolver::advanceStep
 // (src/swe/SweSolver.cpp:803-853), serial path (every ghost is a domain edge). Fusions:
-//   surfbc     enforceSurfBc (:371-384) incl. zero-gradient ghosts
-//   momentum   momentumSource (:386-444)
-//   assemble   shallowwaterRhs + shallowwaterMatCoeff (:446-526)
-//   fixrows    decoupled rows (all off-diagonals 0: dry cells at rest) are solved exactly
+//   momentum   enforceSurfBc (:371-384) incl. zero-gradient ghosts, momentumSource (:386-444)
+//   assemble   shallowwaterRhs + shallowwaterMatCoeff (:446-526); decoupled rows (all off-diagonals 0: dry
+//              cells at rest) are solved exactly
 //   symm       symmetric couplings of the remaining rows, their rhs with decoupled rows folded in
 //   [Krylov]   Jacobi-PCG on the 5-point system (:528-595)
 //   post       enforceSurfBc + cflLimiter + evaprain (:371-384, :597-652); the second
 //              updateDepth of the step is a repeat of the first on the serial path and the
 //              first one's snap finds nothing after evaprain's small-depth removal
-//   depth      updateDepth (:207-304)
-//   dragwtf    updateDragCoef + waterfallLocation (:654-701)
-//   vel        updateVelocity with its limiter pass (:703-770) + enforceVeloBc (:772-778).
+//   depth      updateDepth (:207-304), updateDragCoef + waterfallLocation (:654-701)
+//   vel        updateVelocity with its limiter pass (:703-770) + enforceVeloBc (:772-778), then
+//              updateGeometry (:306-369): a face's velocity reads only its own cell's old geometry.
 //              The limiter only ever sets a face velocity to 0 under conditions on the sign of
 //              that velocity or on its two cells, so its sequential sweep has an order-free
 //              closed form evaluated per face here.
 //   interp     interpVelocity (:780-792), clears cfl_active (:755)
-//   geom       updateGeometry (:306-369)
+// The copies of a step's old fields (etan, un, vn, Vsn) ride with the first kernel that has them at hand. A
+// kernel of its own costs 4 to 5 us of launch at any size up to 512 x 512 (where its work takes 3 to 9 us), so
+// the step is 7 launches and a solve instead of 15.
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -33,7 +34,11 @@ constexpr int NT = 256;
 struct SwK {
   Geo g;
   double dx, dy, dt, gravity, manning, min_depth, visc_x, visc_y, hD, hE, wtfh;
+  // Kernels queued behind a surface solve whose outcome the host has not seen: nonzero when it failed (they
+  // then leave the state alone). Null: run.
+  const int* stop = nullptr;
 };
+__device__ __forceinline__ bool stopped(const SwK& P) { return P.stop != nullptr && *P.stop != 0; }
 
 // src/bc/Polygon.hpp: even-odd ray casting with a +x ray, bounding-box reject, ring closed.
 bool polygon_contains(const double* xy, int n, double x, double y) {
@@ -77,13 +82,20 @@ __device__ inline void ghost_copy(const Geo& g, const C2& t, double* f, double v
   if (t.j == g.ny - 1) f[t.c + g.sy] = v;
 }
 
-__global__ __launch_bounds__(NT) void k_swe_surfbc(SwK P, double* eta, const double* bottom) {
-  const C2 t = cell2(P.g);
-  if (!t.valid) return;
-  double e = eta[t.c];
-  if (e < bottom[t.c]) e = bottom[t.c];
-  eta[t.c] = e;
-  ghost_copy(P.g, t, eta, e);
+// dst = src at this thread's cell and, by the edge threads, at its ghosts and corner ghosts: together the
+// whole field. Call before the thread changes src.
+__device__ inline void copy_cell(const Geo& g, const C2& t, const double* src, double* dst) {
+  const bool w = t.i == 0, e = t.i == g.nx - 1, s = t.j == 0, n = t.j == g.ny - 1;
+  const long long c = t.c, sy = g.sy;
+  dst[c] = src[c];
+  if (w) dst[c - 1] = src[c - 1];
+  if (e) dst[c + 1] = src[c + 1];
+  if (s) dst[c - sy] = src[c - sy];
+  if (n) dst[c + sy] = src[c + sy];
+  if (w && s) dst[c - sy - 1] = src[c - sy - 1];
+  if (e && s) dst[c - sy + 1] = src[c - sy + 1];
+  if (w && n) dst[c + sy - 1] = src[c + sy - 1];
+  if (e && n) dst[c + sy + 1] = src[c + sy + 1];
 }
 
 struct MomIn {
@@ -91,10 +103,17 @@ struct MomIn {
 };
 
 __global__ __launch_bounds__(NT) void k_swe_momentum(SwK P, MomIn m, double* Dx, double* Dy, double* Ex,
-                                                      double* Ey) {
+                                                      double* Ey, double* eta, double* etan, const double* bottom) {
   const C2 t = cell2(P.g);
   if (!t.valid) return;
   const Geo& g = P.g;
+  {  // eta of the last step kept, then clamped to the bed with its ghosts
+    copy_cell(g, t, eta, etan);
+    double e = eta[t.c];
+    if (e < bottom[t.c]) e = bottom[t.c];
+    eta[t.c] = e;
+    ghost_copy(g, t, eta, e);
+  }
   const long long c = t.c, iM = c - 1, iP = c + 1, jM = c - g.sy, jP = c + g.sy;
   const double dx = P.dx, dy = P.dy, dt = P.dt;
   const double u = m.uu[c], v = m.vv[c], vxc = m.vx[c], uyc = m.uy[c];
@@ -129,19 +148,21 @@ __global__ __launch_bounds__(NT) void k_swe_momentum(SwK P, MomIn m, double* Dx,
 }
 
 struct AsmIn {
-  const double *eta, *bottom, *Asz, *Asx, *Asy, *Ex, *Ey, *Vsx, *Vsy, *Dx, *Dy, *dept, *uu, *vv;
+  const double *bottom, *Asz, *Asx, *Asy, *Ex, *Ey, *Vsx, *Vsy, *Dx, *Dy, *dept, *uu, *vv;
 };
 struct AsmOut {
   double *Sxp, *Sxm, *Syp, *Sym, *Sct, *Srhs;
 };
 
-__global__ __launch_bounds__(NT) void k_swe_assemble(SwK P, AsmIn a, AsmOut o, double evap) {
+// A row whose in-domain off-diagonals are all zero is decoupled: x = b / diag exactly (fixed).
+__global__ __launch_bounds__(NT) void k_swe_assemble(SwK P, AsmIn a, AsmOut o, unsigned char* __restrict__ fixed,
+                                                      double* __restrict__ eta, double evap) {
   const C2 t = cell2(P.g);
   if (!t.valid) return;
   const Geo& g = P.g;
   const long long c = t.c, iM = c - 1, jM = c - g.sy;
   const double dt = P.dt, dxdy_x = P.dx, dxdy_y = P.dy;
-  const double e = a.eta[c];
+  const double e = eta[c];
   double rhs = e * a.Asz[c] - dt * (a.Asx[c] * a.Ex[c] - a.Asx[iM] * a.Ex[iM] + a.Asy[c] * a.Ey[c] - a.Asy[jM] * a.Ey[jM]);
   if (e - a.bottom[c] > P.hE) rhs -= evap * a.Asz[c] * dt;
   const double coef = P.gravity * dt * dt;
@@ -177,18 +198,10 @@ __global__ __launch_bounds__(NT) void k_swe_assemble(SwK P, AsmIn a, AsmOut o, d
   o.Sym[c] = sym;
   o.Sct[c] = sct;
   o.Srhs[c] = rhs;
-}
-
-// Rows whose in-domain off-diagonals are all zero are decoupled: x = b / diag exactly.
-__global__ __launch_bounds__(NT) void k_swe_fixrows(SwK P, AsmOut o, unsigned char* fixed, double* eta) {
-  const C2 t = cell2(P.g);
-  if (!t.valid) return;
-  const Geo& g = P.g;
-  const long long c = t.c;
-  const bool fx = (t.i == 0 || o.Sxm[c] == 0.0) && (t.i == g.nx - 1 || o.Sxp[c] == 0.0) &&
-                  (t.j == 0 || o.Sym[c] == 0.0) && (t.j == g.ny - 1 || o.Syp[c] == 0.0);
+  const bool fx = (t.i == 0 || sxm == 0.0) && (t.i == g.nx - 1 || sxp == 0.0) && (t.j == 0 || sym == 0.0) &&
+                  (t.j == g.ny - 1 || syp == 0.0);
   fixed[c] = fx ? 1 : 0;
-  if (fx) eta[c] = o.Srhs[c] / o.Sct[c];
+  if (fx) eta[c] = rhs / sct;
 }
 
 // Symmetric couplings between non-decoupled rows; decoupled neighbours folded into the rhs.
@@ -216,7 +229,7 @@ __global__ __launch_bounds__(NT) void k_swe_symm(SwK P, AsmOut o, const unsigned
 __global__ __launch_bounds__(NT) void k_swe_post(SwK P, double* eta, const double* bottom, const double* dept,
                                                   double* cfl_active, double rain, double evap) {
   const C2 t = cell2(P.g);
-  if (!t.valid) return;
+  if (!t.valid || stopped(P)) return;
   const Geo& g = P.g;
   const long long c = t.c;
   const double b = bottom[c];
@@ -248,10 +261,8 @@ __device__ inline double face_depth(const double* eta, const double* bottom, lon
   return eh - bh;
 }
 
-__global__ __launch_bounds__(NT) void k_swe_depth(SwK P, const double* eta, const double* bottom, double* dept,
-                                                   double* deptx, double* depty) {
-  const C2 t = cell2(P.g);
-  if (!t.valid) return;
+__device__ inline void depth_cell(const SwK& P, const C2& t, const double* eta, const double* bottom, double* dept,
+                                  double* deptx, double* depty) {
   const Geo& g = P.g;
   const long long c = t.c;
   auto dp = [&](long long q) {
@@ -272,14 +283,33 @@ __global__ __launch_bounds__(NT) void k_swe_depth(SwK P, const double* eta, cons
   if (t.i == g.nx - 1) deptx[c + 1] = fmax(face_depth(eta, bottom, c, c + 1), 0.0);
 }
 
-// updateDragCoef + waterfallLocation (SweSolver.cpp:654-701).
-__global__ __launch_bounds__(NT) void k_swe_dragwtf(SwK P, const double* Vs, const double* eta, const double* bXP,
-                                                     const double* bYP, double* CDx, double* CDy, double* wtfx,
-                                                     double* wtfy) {
+// updateDepth, with the last step's Vs kept in Vsn.
+__global__ __launch_bounds__(NT) void k_swe_depth(SwK P, const double* eta, const double* bottom, double* dept,
+                                                   double* deptx, double* depty, const double* Vs, double* Vsn) {
   const C2 t = cell2(P.g);
   if (!t.valid) return;
+  depth_cell(P, t, eta, bottom, dept, deptx, depty);
+  if (Vsn) copy_cell(P.g, t, Vs, Vsn);
+}
+
+struct KeepOld {
+  const double *uu, *vv;
+  double *un, *vn, *Vsn;
+};
+
+// updateDepth, updateDragCoef + waterfallLocation (SweSolver.cpp:654-701), and un, vn, Vsn.
+__global__ __launch_bounds__(NT) void k_swe_depth_drag(SwK P, const double* eta, const double* bottom, double* dept,
+                                                        double* deptx, double* depty, const double* Vs,
+                                                        const double* bXP, const double* bYP, double* CDx, double* CDy,
+                                                        double* wtfx, double* wtfy, KeepOld k) {
+  const C2 t = cell2(P.g);
+  if (!t.valid || stopped(P)) return;
   const Geo& g = P.g;
   const long long c = t.c;
+  depth_cell(P, t, eta, bottom, dept, deptx, depty);
+  copy_cell(g, t, k.uu, k.un);
+  copy_cell(g, t, k.vv, k.vn);
+  copy_cell(g, t, Vs, k.Vsn);
   if (Vs[c] > 0.0) {
     const double coef = P.gravity * P.manning * P.manning;
     const double effh = Vs[c] / (P.dx * P.dy);
@@ -316,56 +346,14 @@ __device__ inline double vel_y(const SwK& P, const VelIn& a, long long c, long l
   return (a.Ey[c] - coef * effhy * (a.eta[c + sy] - a.eta[c])) * a.Dy[c];
 }
 
-__global__ __launch_bounds__(NT) void k_swe_vel(SwK P, VelIn a, VelOut o) {
-  const C2 t = cell2(P.g);
-  if (!t.valid) return;
-  const Geo& g = P.g;
-  const long long c = t.c;
-  const double wt = P.wtfh;
-  // x face between c and c+1
-  double u = vel_x(P, a, c);
-  {
-    bool z = a.Asx[c] < wt * P.dy || a.cfl_active[c] == 1.0 || (u > 0.0 && a.dept[c] < wt);
-    if (t.i + 1 < g.nx) z = z || a.cfl_active[c + 1] == 1.0 || (u < 0.0 && a.dept[c + 1] < wt);
-    if (z) u = 0.0;
-  }
-  double v = vel_y(P, a, c, g.sy);
-  {
-    bool z = a.Asy[c] < wt * P.dx || a.cfl_active[c] == 1.0 || (v > 0.0 && a.dept[c] < wt);
-    if (t.j + 1 < g.ny) z = z || a.cfl_active[c + g.sy] == 1.0 || (v < 0.0 && a.dept[c + g.sy] < wt);
-    if (z) v = 0.0;
-  }
-  o.uu[c] = u;
-  o.vv[c] = v;
-  o.Fu[c] = u * a.Asx[c];
-  o.Fv[c] = v * a.Asy[c];
-  o.cflx[c] = fabs(u * P.dt / P.dx);
-  o.cfly[c] = fabs(v * P.dt / P.dy);
-  ghost_copy(g, t, o.uu, u);
-  ghost_copy(g, t, o.vv, v);
-}
-
-__global__ __launch_bounds__(NT) void k_swe_interp(SwK P, const double* uu, const double* vv, double* uy, double* vx,
-                                                    double* cfl_active) {
-  const C2 t = cell2(P.g);
-  if (!t.valid) return;
-  const Geo& g = P.g;
-  const long long c = t.c;
-  uy[c] = 0.25 * (uu[c] + uu[c - 1] + uu[c + g.sy] + uu[c - 1 + g.sy]);
-  vx[c] = 0.25 * (vv[c] + vv[c - g.sy] + vv[c + 1] + vv[c + 1 - g.sy]);
-  cfl_active[c] = 0.0;
-}
-
 struct GeoOut {
   double *Vs, *Asx, *Asy, *Asz, *Aszx, *Aszy, *Vsx, *Vsy;
 };
 
 // updateGeometry (SweSolver.cpp:306-369): face means read the neighbour's freshly computed
 // value (ghost neighbours: from their own depth, before the ghost fill), then edge ghosts.
-__global__ __launch_bounds__(NT) void k_swe_geom(SwK P, const double* dept, const double* deptx, const double* depty,
-                                                  GeoOut o) {
-  const C2 t = cell2(P.g);
-  if (!t.valid) return;
+__device__ inline void geom_cell(const SwK& P, const C2& t, const double* dept, const double* deptx,
+                                 const double* depty, const GeoOut& o) {
   const Geo& g = P.g;
   const long long c = t.c;
   const double dxdy = P.dx * P.dy;
@@ -395,6 +383,55 @@ __global__ __launch_bounds__(NT) void k_swe_geom(SwK P, const double* dept, cons
     o.Vsx[c - 1] = Vs;
     o.Aszx[c - 1] = Asz;
   }
+}
+
+__global__ __launch_bounds__(NT) void k_swe_geom(SwK P, const double* dept, const double* deptx, const double* depty,
+                                                  GeoOut o) {
+  const C2 t = cell2(P.g);
+  if (t.valid) geom_cell(P, t, dept, deptx, depty, o);
+}
+
+// The velocities (from the old geometry of the thread's own cell), then that cell's new geometry.
+__global__ __launch_bounds__(NT) void k_swe_vel(SwK P, VelIn a, VelOut o, const double* deptx, const double* depty,
+                                                 GeoOut go) {
+  const C2 t = cell2(P.g);
+  if (!t.valid || stopped(P)) return;
+  const Geo& g = P.g;
+  const long long c = t.c;
+  const double wt = P.wtfh;
+  // x face between c and c+1
+  double u = vel_x(P, a, c);
+  {
+    bool z = a.Asx[c] < wt * P.dy || a.cfl_active[c] == 1.0 || (u > 0.0 && a.dept[c] < wt);
+    if (t.i + 1 < g.nx) z = z || a.cfl_active[c + 1] == 1.0 || (u < 0.0 && a.dept[c + 1] < wt);
+    if (z) u = 0.0;
+  }
+  double v = vel_y(P, a, c, g.sy);
+  {
+    bool z = a.Asy[c] < wt * P.dx || a.cfl_active[c] == 1.0 || (v > 0.0 && a.dept[c] < wt);
+    if (t.j + 1 < g.ny) z = z || a.cfl_active[c + g.sy] == 1.0 || (v < 0.0 && a.dept[c + g.sy] < wt);
+    if (z) v = 0.0;
+  }
+  o.uu[c] = u;
+  o.vv[c] = v;
+  o.Fu[c] = u * a.Asx[c];
+  o.Fv[c] = v * a.Asy[c];
+  o.cflx[c] = fabs(u * P.dt / P.dx);
+  o.cfly[c] = fabs(v * P.dt / P.dy);
+  ghost_copy(g, t, o.uu, u);
+  ghost_copy(g, t, o.vv, v);
+  geom_cell(P, t, a.dept, deptx, depty, go);
+}
+
+__global__ __launch_bounds__(NT) void k_swe_interp(SwK P, const double* uu, const double* vv, double* uy, double* vx,
+                                                    double* cfl_active) {
+  const C2 t = cell2(P.g);
+  if (!t.valid || stopped(P)) return;
+  const Geo& g = P.g;
+  const long long c = t.c;
+  uy[c] = 0.25 * (uu[c] + uu[c - 1] + uu[c + g.sy] + uu[c - 1 + g.sy]);
+  vx[c] = 0.25 * (vv[c] + vv[c - g.sy] + vv[c + 1] + vv[c + 1 - g.sy]);
+  cfl_active[c] = 0.0;
 }
 
 // PolygonBC::applySurface (src/bc/PolygonBC.cpp:16-78): each interior cell tagged with a region
@@ -473,12 +510,6 @@ const char* kNames[] = {"eta",  "etan", "bottom", "bottomXP", "bottomYP", "dept"
                         "Asz",  "Aszx", "Aszy",   "Vsx",      "Vsy",      "CDx",  "CDy",   "Dx",    "Dy",
                         "Ex",   "Ey",   "cflx",   "cfly",     "Fu",       "Fv",   "Sxp",   "Sxm",   "Syp",
                         "Sym",  "Sct",  "Srhs",   "cfl_active", "wtfx",   "wtfy"};
-
-__global__ __launch_bounds__(NT) void k_copy_field(const double* __restrict__ src, double* __restrict__ dst,
-                                                   long long n) {
-  const long long c = (long long)blockIdx.x * NT + threadIdx.x;
-  if (c < n) dst[c] = src[c];
-}
 
 }  // namespace
 
@@ -653,7 +684,8 @@ void SweState::initialize_eta(const double* eta_phys, double init_eta) {
   }
   const SwK P = make_swk(g_, dx_, dy_, p_);
   const dim3 grid(ceil_div(nx, 64), ceil_div(ny, 4)), blk(NT);
-  hipLaunchKernelGGL(k_swe_depth, grid, blk, 0, s_, P, f_["eta"], f_["bottom"], f_["dept"], f_["deptx"], f_["depty"]);
+  hipLaunchKernelGGL(k_swe_depth, grid, blk, 0, s_, P, f_["eta"], f_["bottom"], f_["dept"], f_["deptx"], f_["depty"],
+                     nullptr, nullptr);
   FREHG_LAUNCH_CHECK();
   GeoOut go{f_["Vs"], f_["Asx"], f_["Asy"], f_["Asz"], f_["Aszx"], f_["Aszy"], f_["Vsx"], f_["Vsy"]};
   hipLaunchKernelGGL(k_swe_geom, grid, blk, 0, s_, P, f_["dept"], f_["deptx"], f_["depty"], go);
@@ -672,54 +704,40 @@ void SweState::enq_pre(double evap) {
   const SwK P = make_swk(g_, dx_, dy_, p_);
   const dim3 grid(ceil_div(g_.nx, 64), ceil_div(g_.ny, 4)), blk(NT);
   auto F = [&](const char* nm) { return f_[nm]; };
-  copy_field(F("eta"), F("etan"));
-  hipLaunchKernelGGL(k_swe_surfbc, grid, blk, 0, s_, P, F("eta"), F("bottom"));
-  FREHG_LAUNCH_CHECK();
   MomIn m{F("uu"), F("vv"), F("vx"), F("uy"), F("cflx"), F("cfly"), F("Vsx"), F("Vsy"),
           F("Asx"), F("Asy"), F("Aszx"), F("Aszy"), F("CDx"), F("CDy")};
-  hipLaunchKernelGGL(k_swe_momentum, grid, blk, 0, s_, P, m, F("Dx"), F("Dy"), F("Ex"), F("Ey"));
+  hipLaunchKernelGGL(k_swe_momentum, grid, blk, 0, s_, P, m, F("Dx"), F("Dy"), F("Ex"), F("Ey"), F("eta"), F("etan"),
+                     F("bottom"));
   FREHG_LAUNCH_CHECK();
-  AsmIn a{F("eta"), F("bottom"), F("Asz"), F("Asx"), F("Asy"), F("Ex"), F("Ey"), F("Vsx"),
+  AsmIn a{F("bottom"), F("Asz"), F("Asx"), F("Asy"), F("Ex"), F("Ey"), F("Vsx"),
           F("Vsy"), F("Dx"),     F("Dy"),  F("dept"), F("uu"), F("vv")};
   AsmOut o{F("Sxp"), F("Sxm"), F("Syp"), F("Sym"), F("Sct"), F("Srhs")};
-  hipLaunchKernelGGL(k_swe_assemble, grid, blk, 0, s_, P, a, o, evap);
-  FREHG_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_swe_fixrows, grid, blk, 0, s_, P, o, fixed_, F("eta"));
+  hipLaunchKernelGGL(k_swe_assemble, grid, blk, 0, s_, P, a, o, fixed_, F("eta"), evap);
   FREHG_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_swe_symm, grid, blk, 0, s_, P, o, fixed_, F("eta"), ax_, ay_, b_);
   FREHG_LAUNCH_CHECK();
 }
 
-// Kernels of the step after the surface solve: depth, drag and wet/dry faces, velocities,
-// their interpolation and the surface geometry for the next step.
-void SweState::enq_post(double rain, double evap) {
-  const SwK P = make_swk(g_, dx_, dy_, p_);
+// Kernels of the step after the surface solve: depth, drag and wet/dry faces, velocities with the surface
+// geometry for the next step, and their interpolation; with `stop` they do nothing behind a failed solve.
+void SweState::enq_post(double rain, double evap, const int* stop) {
+  SwK P = make_swk(g_, dx_, dy_, p_);
+  P.stop = stop;
   const dim3 grid(ceil_div(g_.nx, 64), ceil_div(g_.ny, 4)), blk(NT);
   auto F = [&](const char* nm) { return f_[nm]; };
   hipLaunchKernelGGL(k_swe_post, grid, blk, 0, s_, P, F("eta"), F("bottom"), F("dept"), F("cfl_active"), rain, evap);
   FREHG_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_swe_depth, grid, blk, 0, s_, P, F("eta"), F("bottom"), F("dept"), F("deptx"), F("depty"));
+  KeepOld k{F("uu"), F("vv"), F("un"), F("vn"), F("Vsn")};
+  hipLaunchKernelGGL(k_swe_depth_drag, grid, blk, 0, s_, P, F("eta"), F("bottom"), F("dept"), F("deptx"), F("depty"),
+                     F("Vs"), F("bottomXP"), F("bottomYP"), F("CDx"), F("CDy"), F("wtfx"), F("wtfy"), k);
   FREHG_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_swe_dragwtf, grid, blk, 0, s_, P, F("Vs"), F("eta"), F("bottomXP"), F("bottomYP"), F("CDx"),
-                     F("CDy"), F("wtfx"), F("wtfy"));
-  FREHG_LAUNCH_CHECK();
-  copy_field(F("uu"), F("un"));
-  copy_field(F("vv"), F("vn"));
   VelIn vi{F("Ex"), F("Ey"), F("Dx"), F("Dy"), F("Vsx"), F("Vsy"), F("Asx"), F("Asy"), F("eta"), F("dept"),
            F("cfl_active")};
   VelOut vo{F("uu"), F("vv"), F("Fu"), F("Fv"), F("cflx"), F("cfly")};
-  hipLaunchKernelGGL(k_swe_vel, grid, blk, 0, s_, P, vi, vo);
+  GeoOut go{F("Vs"), F("Asx"), F("Asy"), F("Asz"), F("Aszx"), F("Aszy"), F("Vsx"), F("Vsy")};
+  hipLaunchKernelGGL(k_swe_vel, grid, blk, 0, s_, P, vi, vo, F("deptx"), F("depty"), go);
   FREHG_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_swe_interp, grid, blk, 0, s_, P, F("uu"), F("vv"), F("uy"), F("vx"), F("cfl_active"));
-  FREHG_LAUNCH_CHECK();
-  copy_field(F("Vs"), F("Vsn"));
-  GeoOut go{F("Vs"), F("Asx"), F("Asy"), F("Asz"), F("Aszx"), F("Aszy"), F("Vsx"), F("Vsy")};
-  hipLaunchKernelGGL(k_swe_geom, grid, blk, 0, s_, P, F("dept"), F("deptx"), F("depty"), go);
-  FREHG_LAUNCH_CHECK();
-}
-
-void SweState::copy_field(const double* src, double* dst) {
-  hipLaunchKernelGGL(k_copy_field, dim3(ceil_div(n_, NT)), dim3(NT), 0, s_, src, dst, n_);
   FREHG_LAUNCH_CHECK();
 }
 
@@ -756,7 +774,7 @@ void SweState::step(double rain, double evap, frehg_solve_stats* st) {
         FREHG_HIP(hipGraphDestroy(g));
       };
       capture(&graph_pre_, [&] { enq_pre(evap); });
-      capture(&graph_post_, [&] { enq_post(rain, evap); });
+      capture(&graph_post_, [&] { enq_post(rain, evap, nullptr); });
       graph_rain_ = rain;
       graph_evap_ = evap;
       graph_params_ = p_;
@@ -765,9 +783,19 @@ void SweState::step(double rain, double evap, frehg_solve_stats* st) {
   } else {
     enq_pre(evap);
   }
-  sr = kry_->solve(A, nullptr, b_, f_["Srhs"], f_["eta"], fixed_, true, false, kc);
-  if (use_graph_) FREHG_HIP(hipGraphLaunch(graph_post_, s_));
-  else enq_post(rain, evap);
+  // A solve that is one launch is queued, and the kernels behind it with it: their launches then run while it
+  // does. They watch its outcome on the device, so a solve that fails leaves the state as if it had been
+  // waited for.
+  const bool queued = !use_graph_ && kry_->enqueue(A, b_, f_["Srhs"], f_["eta"], fixed_, true, kc);
+  if (queued) {
+    enq_post(rain, evap, kry_->failed_flag());
+    FREHG_HIP(hipStreamSynchronize(s_));
+  }
+  if (!queued || !kry_->finish_queued(&sr)) {
+    sr = kry_->solve(A, nullptr, b_, f_["Srhs"], f_["eta"], fixed_, true, false, kc);
+    if (use_graph_) FREHG_HIP(hipGraphLaunch(graph_post_, s_));
+    else enq_post(rain, evap, nullptr);
+  }
   if (st) {
     std::memset(st, 0, sizeof(*st));
     st->iterations = sr.iterations;
@@ -832,9 +860,9 @@ void SweState::apply_boundaries_async(double dt) {
                      f_["eta"], (const double*)f_["bottom"], bcpart_);
   FREHG_LAUNCH_CHECK();
   // depth and geometry refresh (PolygonBC.cpp:74-77); updateGeometry first keeps Vs as Vsn
-  hipLaunchKernelGGL(k_swe_depth, grid, blk, 0, s_, P, f_["eta"], f_["bottom"], f_["dept"], f_["deptx"], f_["depty"]);
+  hipLaunchKernelGGL(k_swe_depth, grid, blk, 0, s_, P, f_["eta"], f_["bottom"], f_["dept"], f_["deptx"], f_["depty"],
+                     (const double*)f_["Vs"], f_["Vsn"]);
   FREHG_LAUNCH_CHECK();
-  copy_field(f_["Vs"], f_["Vsn"]);
   GeoOut go{f_["Vs"], f_["Asx"], f_["Asy"], f_["Asz"], f_["Aszx"], f_["Aszy"], f_["Vsx"], f_["Vsy"]};
   hipLaunchKernelGGL(k_swe_geom, grid, blk, 0, s_, P, f_["dept"], f_["deptx"], f_["depty"], go);
   FREHG_LAUNCH_CHECK();

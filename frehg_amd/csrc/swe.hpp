@@ -57,8 +57,7 @@ class SweState {
   void set_raw(const std::string& name, const double* src);
   void get_raw(const std::string& name, double* dst);
   void enq_pre(double evap);
-  void enq_post(double rain, double evap);
-  void copy_field(const double* src, double* dst);
+  void enq_post(double rain, double evap, const int* stop);
 
   Geo g_;  // nz = 1; 2D index = sidx
   double dx_, dy_;
