@@ -1054,7 +1054,8 @@ Krylov::Krylov(const Geo& g, bool three_d, hipStream_t stream, Profiler* prof, c
   part_ = ws.part;
   part_u_ = ws.part_u;
   ctl_ = ws.ctl;
-  host_ctl_ = host_ctl_own_;
+  host_ctl_ = ws.host ? ws.host : host_ctl_own_;
+  host_out_ = ws.host != nullptr;
   // the resident solve needs none of the CG vectors: its exchange buffers take their place
   double* words[4] = {r_, z_, p0_, p1_};
   for (int q = 0; q < 4; ++q) halo_[q] = reinterpret_cast<unsigned long long*>(words[q]);
@@ -1525,13 +1526,13 @@ void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T
   a.fixed = fixed;
   a.r0 = r0;
   a.ctl = started;
-  // the outcome goes straight to pinned host memory (a borrowed workspace has none: resident_wait copies it)
-  KrylovCtl* out = borrowed_ ? ctl_ : host_ctl_;
+  // the outcome goes straight to pinned host memory (a borrowed workspace may have none: copied by the caller)
+  KrylovCtl* out = host_out_ ? host_ctl_ : ctl_;
   host_ctl_[1].iters = 0;
   a.out = out;
   a.timeout = &out[1].iters;
   a.failed = failed_flag();
-  if (failed_dirty_) FREHG_HIP(hipMemsetAsync(a.failed, 0, sizeof(int), s_));
+  if (failed_dirty_ && !borrowed_) FREHG_HIP(hipMemsetAsync(a.failed, 0, sizeof(int), s_));  // (borrowed: cleared)
   failed_dirty_ = true;  // until its outcome has been seen
   a.rtol = rtol;
   a.atol = atol;
@@ -1584,14 +1585,14 @@ template <typename T>
 bool Krylov::cg_resident(const StencilView<T>& A, const T* b, const T* bn, T* x, const unsigned char* fixed, bool zero,
                          bool guard, double rtol, double atol, int max_it, const T* r0, const KrylovCtl* started) {
   resident_launch<T>(A, b, bn, x, fixed, zero, guard, rtol, atol, max_it, r0, started);
-  if (borrowed_) FREHG_HIP(hipMemcpyAsync(host_ctl_, ctl_, 2 * sizeof(KrylovCtl), hipMemcpyDeviceToHost, s_));
+  if (!host_out_) FREHG_HIP(hipMemcpyAsync(host_ctl_, ctl_, 2 * sizeof(KrylovCtl), hipMemcpyDeviceToHost, s_));
   FREHG_HIP(hipStreamSynchronize(s_));
   return resident_ended();
 }
 
 bool Krylov::enqueue(const StencilView<double>& A, const double* b, const double* bn, double* x,
                      const unsigned char* fixed, bool x0_zero, const KrylovConfig& cfg) {
-  if (cfg.ksp != FREHG_KSP_CG || cfg.precision != 0 || borrowed_ || !resident(0) || !A.symmetric()) return false;
+  if (cfg.ksp != FREHG_KSP_CG || cfg.precision != 0 || !host_out_ || !resident(0) || !A.symmetric()) return false;
   resident_launch<double>(A, b, bn, x, fixed, x0_zero, false, cfg.rtol, cfg.atol, cfg.max_it, nullptr, nullptr);
   return true;
 }

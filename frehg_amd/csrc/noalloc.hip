@@ -37,14 +37,13 @@ namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_setup_mu;
 void* g_scratch_ptr[kMaxDevices] = {};  // device address of `scratch`, per device
+KrylovCtl* g_host_ctl[kMaxDevices] = {};  // pinned results of a call, per device
 std::mutex g_call_mu[kMaxDevices];      // serialises this process's calls per device
 
 constexpr int NT = 256;
 
-// Fill kernel (no hipMemsetAsync, so a caller may also capture the call's launches): the CG vectors or
-// exchange buffers, and the flag word.
-__global__ __launch_bounds__(NT) void k_na_zero(double* a, long long n, int* flags) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *flags = 0;
+// Fill kernel (no hipMemsetAsync, so a caller may also capture the call's launches).
+__global__ __launch_bounds__(NT) void k_na_zero(double* a, long long n) {
   for (long long c = (long long)blockIdx.x * NT + threadIdx.x; c < n; c += (long long)gridDim.x * NT) a[c] = 0.0;
 }
 
@@ -58,8 +57,15 @@ struct NaOperator {
 // arrays (3D rows z-fastest, 2D rows x-fastest), zero elsewhere (ghosts, pitch padding, faces on
 // the domain edge). flags: bit 0 = a +face coupling differs from its neighbour's -face coupling
 // (CG needs a symmetric operator), bit 1 = a zero or non-finite diagonal.
+// (the operators of one-block resident solves and of 2D; larger 3D ones take k_na_pack3). *failed is the word
+// that the solve sets for the unpack kernel; a bad row sets it too, unless this kernel is the one to clear it.
+__device__ inline void na_bad(int* flags, int* failed, int bad) {
+  __hip_atomic_fetch_or(flags, bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);  // pinned host memory
+  if (failed) __hip_atomic_store(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __global__ __launch_bounds__(NT) void k_na_pack(Geo g, int three, NaOperator op, long long n, double* D, double* ax,
-                                                double* ay, double* az, double* b, double* x, int* flags) {
+                                                double* ay, double* az, double* b, double* x, int* flags, int* failed, int clear) {
+  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *failed = 0;
   const long long c = (long long)blockIdx.x * NT + threadIdx.x;
   if (c >= n) return;
   const int nz = three ? g.nz : 1;
@@ -89,7 +95,7 @@ __global__ __launch_bounds__(NT) void k_na_pack(Geo g, int three, NaOperator op,
     vx = plus(0, ii < g.nx - 1, three ? r + nz : r + 1);
     vy = plus(1, j < g.ny - 1, three ? r + (long long)g.nx * nz : r + g.nx);
     if (three) vz = plus(2, k < nz - 1, r + 1);
-    if (bad) atomicOr(flags, bad);
+    if (bad) na_bad(flags, clear ? nullptr : failed, bad);
   }
   D[c] = d;
   ax[c] = vx;
@@ -99,7 +105,52 @@ __global__ __launch_bounds__(NT) void k_na_pack(Geo g, int three, NaOperator op,
   x[c] = 0.0;
 }
 
-__global__ __launch_bounds__(NT) void k_na_unpack(Geo g, int three, const double* x, double* x_owned) {
+// The interior rows of a 3D operator through LDS: tiles of 32 cells in x by 32 layers of one row j, read along
+// z (the owned order) and written along x. The rest of the padded arrays was cleared before. Reading along x
+// took 74 us at 128 x 96 x 48 (each 64-byte line of the eight inputs fetched once per layer it holds).
+constexpr int kPt = 32;
+__global__ __launch_bounds__(NT) void k_na_pack3(Geo g, NaOperator op, double* D, double* ax, double* ay, double* az,
+                                                 double* b, int* flags, int* failed) {
+  __shared__ double lds[5][kPt][kPt + 1];
+  const int j = blockIdx.x, i0 = blockIdx.y * kPt, k0 = blockIdx.z * kPt;
+  const int u = threadIdx.x & (kPt - 1), v0 = threadIdx.x / kPt;
+  int bad = 0;
+  for (int v = v0; v < kPt; v += NT / kPt) {
+    const int i = i0 + v, k = k0 + u;
+    if (i >= g.nx || k >= g.nz) continue;
+    const long long r = ((long long)j * g.nx + i) * g.nz + k;
+    const double d = op.diag[r];
+    if (!(d != 0.0 && isfinite(d))) bad |= 2;
+    auto plus = [&](int dir, bool inside, long long rn) {
+      if (!inside) return 0.0;
+      const double a = op.off[2 * dir + 1][r], back = op.off[2 * dir][rn];
+      if (fabs(a - back) > 1e-12 * (fabs(a) + fabs(back))) bad |= 1;
+      return a;
+    };
+    lds[0][u][v] = d;
+    lds[1][u][v] = plus(0, i < g.nx - 1, r + g.nz);
+    lds[2][u][v] = plus(1, j < g.ny - 1, r + (long long)g.nx * g.nz);
+    lds[3][u][v] = plus(2, k < g.nz - 1, r + 1);
+    lds[4][u][v] = op.b[r];
+  }
+  if (bad) na_bad(flags, failed, bad);
+  __syncthreads();
+  for (int v = v0; v < kPt; v += NT / kPt) {
+    const int i = i0 + u, k = k0 + v;
+    if (i >= g.nx || k >= g.nz) continue;
+    const long long c = g.idx(i, j, k);
+    D[c] = lds[0][v][u];
+    ax[c] = lds[1][v][u];
+    ay[c] = lds[2][v][u];
+    az[c] = lds[3][v][u];
+    b[c] = lds[4][v][u];
+  }
+}
+
+// x to the owned order, unless the solve before failed.
+__global__ __launch_bounds__(NT) void k_na_unpack(Geo g, int three, const double* x, double* x_owned,
+                                                  const int* failed, const int* flags) {
+  if ((failed && *failed) || (flags && *flags)) return;
   const int nz = three ? g.nz : 1;
   const long long r = (long long)blockIdx.x * NT + threadIdx.x;
   if (r >= (long long)g.nx * g.ny * nz) return;
@@ -130,6 +181,12 @@ void noalloc_setup(int device) {
   const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
   if (e != hipSuccess || ptr == nullptr)
     throw HipError(std::string("hipGetSymbolAddress(scratch) failed: ") + hipGetErrorString(e));
+  // results of a call, written by its kernels: two control blocks and the flag word (held, as the scratch
+  // array is, until the process ends)
+  void* host = nullptr;
+  if (hipHostMalloc(&host, 3 * sizeof(KrylovCtl), hipHostMallocDefault) != hipSuccess || host == nullptr)
+    throw HipError("hipHostMalloc for the allocation-free solve failed");
+  g_host_ctl[device] = static_cast<KrylovCtl*>(host);
   g_scratch_ptr[device] = ptr;
 }
 
@@ -170,38 +227,58 @@ void ls_solve_noalloc(int device, hipStream_t s, int ndim, int nx, int ny, int n
   double* az = three ? reinterpret_cast<double*>(take((size_t)n * sizeof(double))) : nullptr;
   double* b = reinterpret_cast<double*>(take((size_t)n * sizeof(double)));
   double* x = reinterpret_cast<double*>(take((size_t)n * sizeof(double)));
-  int* flags = reinterpret_cast<int*>(take(sizeof(int)));
-  const KrylovWorkspace ws = Krylov::carve_workspace(base, g, three);
+  (void)take(sizeof(int));
+  KrylovWorkspace ws = Krylov::carve_workspace(base, g, three);
+  ws.host = g_host_ctl[device];
+  int* flags = &ws.host[2].iters;
+  *flags = 0;
   Profiler off;  // no timing events (they would be created on first use)
   Krylov kry(g, three, s, &off, ws);
-  // CG vectors from earlier calls hold other geometries: clear them (their ghost entries meet zero
-  // coefficients and must be finite; for the resident solve, which keeps its vectors on the compute
-  // units, they are exchange buffers whose words must not carry a tag) with the control blocks behind
-  // them, and the flag word. A resident solve of one block exchanges nothing.
-  double* z0 = kry.resident_blocks(0) == 1 ? reinterpret_cast<double*>(ws.ctl) : ws.r;
-  const long long zn = (reinterpret_cast<char*>(ws.ctl + 3) - reinterpret_cast<char*>(z0)) / (long long)sizeof(double);
-  hipLaunchKernelGGL(k_na_zero, dim3((unsigned)std::min<long long>(4096, (zn + NT - 1) / NT)), dim3(NT), 0, s, z0, zn,
-                     flags);
-  FREHG_LAUNCH_CHECK();
   NaOperator op{};
   op.diag = diag;
   for (int d = 0; d < ndir; ++d) op.off[d] = offdiag[d];
   op.b = b_owned;
-  hipLaunchKernelGGL(k_na_pack, dim3(ceil_div(n, NT)), dim3(NT), 0, s, g, three ? 1 : 0, op, n, D, ax, ay, az, b, x,
-                     flags);
+  // CG vectors from earlier calls hold other geometries: clear them (their ghost entries meet zero
+  // coefficients and must be finite; for the resident solve, which keeps its vectors on the compute
+  // units, they are exchange buffers whose words must not carry a tag) with the control blocks behind
+  // them. A resident solve of one block exchanges nothing.
+  const bool one = kry.resident_blocks(0) == 1, tiled = three && !one;
+  auto zero = [&](double* from, void* to) {
+    const long long zn = (reinterpret_cast<char*>(to) - reinterpret_cast<char*>(from)) / (long long)sizeof(double);
+    hipLaunchKernelGGL(k_na_zero, dim3((unsigned)std::min<long long>(4096, (zn + NT - 1) / NT)), dim3(NT), 0, s, from,
+                       zn);
+    FREHG_LAUNCH_CHECK();
+  };
+  if (!one) zero(tiled ? D : ws.r, ws.ctl + 3);
+  if (tiled)
+    hipLaunchKernelGGL(k_na_pack3, dim3(ny, ceil_div(nx, kPt), ceil_div(nz, kPt)), dim3(NT), 0, s, g, op, D, ax, ay, az,
+                       b, flags, kry.failed_flag());
+  else
+    hipLaunchKernelGGL(k_na_pack, dim3(ceil_div(n, NT)), dim3(NT), 0, s, g, three ? 1 : 0, op, n, D, ax, ay, az, b, x,
+                       flags, kry.failed_flag(), one ? 1 : 0);
   FREHG_LAUNCH_CHECK();
-  int hflags = 0;
-  FREHG_HIP(hipMemcpyAsync(&hflags, flags, sizeof(int), hipMemcpyDeviceToHost, s));
+  const StencilView<double> A{D, ax, ay, az};
+  const long long rows = (long long)nx * ny * (three ? nz : 1);
+  auto unpack = [&](const int* failed) {
+    hipLaunchKernelGGL(k_na_unpack, dim3(ceil_div(rows, NT)), dim3(NT), 0, s, g, three ? 1 : 0, (const double*)x,
+                       x_owned, failed, failed && one ? flags : nullptr);
+    FREHG_LAUNCH_CHECK();
+  };
+  // A one-launch solve is queued with the unpack kernel behind it and the call waits once; the checks of the
+  // operator are looked at before the solve's outcome, so they are reported as before.
+  const bool queued = kry.enqueue(A, b, nullptr, x, nullptr, true, kc);
+  if (queued) unpack(kry.failed_flag());
   FREHG_HIP(hipStreamSynchronize(s));
+  const int hflags = *flags;
   if (hflags & 2) throw ArgError("frehg_ls_solve_noalloc: zero diagonal (Jacobi needs D != 0)");
   if (hflags & 1) throw ArgError("frehg_ls_solve_noalloc: operator is not symmetric (CG requires A = A^T)");
-  const StencilView<double> A{D, ax, ay, az};
-  const SolveResult sr = kry.solve(A, nullptr, b, nullptr, x, nullptr, true, false, kc);
-  const long long rows = (long long)nx * ny * (three ? nz : 1);
-  hipLaunchKernelGGL(k_na_unpack, dim3(ceil_div(rows, NT)), dim3(NT), 0, s, g, three ? 1 : 0, (const double*)x,
-                     x_owned);
-  FREHG_LAUNCH_CHECK();
-  FREHG_HIP(hipStreamSynchronize(s));
+  SolveResult sr;
+  if (!queued || !kry.finish_queued(&sr)) {
+    if (queued) zero(ws.r, ws.ctl + 3);  // the exchange buffers become CG vectors again
+    sr = kry.solve(A, nullptr, b, nullptr, x, nullptr, true, false, kc);
+    unpack(nullptr);
+    FREHG_HIP(hipStreamSynchronize(s));
+  }
   if (st) {
     std::memset(st, 0, sizeof(*st));
     st->iterations = sr.iterations;

@@ -91,3 +91,30 @@ def test_noalloc_rejects_what_it_does_not_serve():
     with pytest.raises(gpu.FrehgError) as e:
         _solve_noalloc(ctx, 3, 8, 7, 6, diag, offs, b, abi.solver_config(1e-10))
     assert "symmetric" in str(e.value)
+
+
+@pytest.mark.parametrize("ndim,nx,ny,nz", [(3, 33, 5, 65), (3, 32, 40, 3), (3, 1, 70, 31), (2, 45, 50, 1), (3, 9, 8, 7)])
+def test_noalloc_leaves_the_solution_alone_on_a_bad_operator(ndim, nx, ny, nz):
+    """Zero diagonals and nonsymmetric couplings are found while the operator is packed (tiles of 32 x 32 in x and
+    z, their remainders, and the untiled forms) and reported, with x untouched; the next call is served."""
+    ctx = gpu.Context(0)
+    diag, offs, b = spd_stencil(ndim, nx, ny, nz, 6)
+    cfg = abi.solver_config(1e-11)
+    ref, _ = ctx.ls_solve(ndim, nx, ny, nz, diag, offs, b, cfg)
+    for what in ("diagonal", "symmetric"):
+        d, o = diag.copy(), [v.copy() for v in offs]
+        if what == "diagonal":
+            d[-1] = 0.0
+        else:
+            o[3][np.flatnonzero(o[3])[-1]] *= 1.5
+        dd, oo, bb = _dev(d), [_dev(v) for v in o], _dev(b)
+        x = torch.full_like(bb, 7.0)
+        torch.cuda.synchronize()
+        with pytest.raises(gpu.FrehgError) as e:
+            ctx.ls_solve_noalloc(ndim, nx, ny, nz, dd.data_ptr(), [v.data_ptr() for v in oo], bb.data_ptr(),
+                                 x.data_ptr(), cfg)
+        assert e.value.code == abi.ERR_INVALID_ARG and what in str(e.value)
+        assert bool((x == 7.0).all())
+        x, st = _solve_noalloc(ctx, ndim, nx, ny, nz, diag, offs, b, cfg)
+        assert st.converged
+        np.testing.assert_allclose(x, ref, rtol=0, atol=1e-8 * np.abs(ref).max())
