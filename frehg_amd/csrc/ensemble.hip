@@ -1,8 +1,9 @@
 // Batched ensemble of independent Richards boxes (see ensemble.hpp).
 //
-// Tile spaces: "cell" tiles are 64 x 4 columns of one layer (ntx * nty * nz per box); "SpMV"
-// tiles are 64 x 4 columns of kc layers. A launch covers the tiles of every box; block -> tile goes
-// through xcd_remap (neighbouring tiles share an XCD) and tile -> box through a prefix table.
+// Tile spaces: a tile is 256 columns of a box, taken along its rows one after the other: "cell" tiles
+// are one layer deep (ncol * nz per box), "SpMV" tiles kc layers. A launch covers the tiles of every
+// box; block -> tile goes through xcd_remap (neighbouring tiles share an XCD) and tile -> box through
+// a prefix table.
 // Per-block partial sums are indexed by tile, so the partials of one box are contiguous and a
 // one-block-per-box kernel reduces them in a fixed order.
 //
@@ -24,11 +25,12 @@ namespace {
 
 using namespace redev;
 constexpr int NT = kReNT;
+constexpr int kRowPad = 8;  // lanes: see tile_column
 constexpr int NSUM = 6;  // ledger partials per tile: before, storage, boundary, after, adjust, max dh
 
 struct Pools {
   double *h, *hn, *wc, *wcn, *wch, *hwc, *ch, *kr, *Kx, *Ky, *Kz, *qx, *qy, *qz, *D, *ax, *ay, *az, *rhs;
-  // extrapolated start only: the post-solve head of the last step, then the start of the next
+  // extrapolated start only: the post-solve head of the last step
   double* hp = nullptr;
 };
 
@@ -42,33 +44,26 @@ __device__ __forceinline__ int find_box(const unsigned int* t0, int nbox, unsign
   return lo;
 }
 
-// Box and cell of this thread in a cell-tile launch.
-struct BoxCell {
-  int b;
-  unsigned int tile;
-  long long off;
-  ReK P;
-  Cell t;
-};
-
-__device__ __forceinline__ BoxCell box_cell(const EnsBox* boxes, const unsigned int* t0, int nbox) {
-  BoxCell r;
-  r.tile = xcd_remap(blockIdx.x, gridDim.x);
-  r.b = find_box(t0, nbox, r.tile);
-  const EnsBox& B = boxes[r.b];
-  r.P = B.P;
-  r.off = B.off;
-  const unsigned int local = r.tile - t0[r.b];
-  const unsigned int bx = local % B.ntx, rest = local / B.ntx;
-  r.t = cell_at(r.P.g, bx, rest % B.nty, rest / B.nty);
-  return r;
+// Column (i, j) of this thread in tile `col` of a layer of box B; false outside of it. The tiles take the
+// rows one after the other, each padded to nxp lanes so that a row starts on a 64-byte boundary.
+// Tiles of 64 x 4 columns left 28 % of the lanes of 24 boxes of 32 to 128 columns idle, these 4 %
+// (MI355X, 12.6 M cells: FP32 SpMV 28.6 -> 24.6 us, residual sweep 220 -> 187, assembly 405 -> 350,
+// fluxes and corrector 566 -> 490). Rows padded to 1 or 16 lanes: 1 and 2 % slower steps. Cell tiles
+// of up to 8 layers, which share the search for the box and its parameters, gave no more: in a loop
+// the van Genuchten relations take 124 registers instead of 71.
+__device__ __forceinline__ bool tile_column(const EnsBox& B, unsigned int col, int& i, int& j) {
+  const unsigned int p = col * NT + threadIdx.x;
+  j = (int)(p / (unsigned int)B.nxp);
+  i = (int)(p - (unsigned int)j * (unsigned int)B.nxp);
+  return i < B.P.g.nx && j < B.P.g.ny;
 }
 
-// box_cell with the box parameters in soil variant K (see with_soil_variant_code) and the tile
-// order of the single-box kernels: ZF = 1 takes the layer fastest within the box's tiles (the
-// layers above and below a tile were just read through the same L2), ZF = 0 x fastest.
+// Box and cell of this thread in a cell-tile launch, with the box parameters in soil variant K (see
+// with_soil_variant_code) and the tile order of the single-box kernels: ZF = 1 takes the layer fastest
+// within the box's tiles (the layers above and below a tile were just read through the same L2),
+// ZF = 0 the columns.
 template <class K>
-struct BoxCellT {
+struct BoxCell {
   int b;
   unsigned int tile;
   long long off;
@@ -77,27 +72,18 @@ struct BoxCellT {
 };
 
 template <class K, int ZF>
-__device__ __forceinline__ BoxCellT<K> box_cell_as(const EnsBox* boxes, const unsigned int* t0, int nbox) {
-  BoxCellT<K> r;
+__device__ __forceinline__ BoxCell<K> box_cell(const EnsBox* boxes, const unsigned int* t0, int nbox) {
+  BoxCell<K> r;
   r.tile = xcd_remap(blockIdx.x, gridDim.x);
   r.b = find_box(t0, nbox, r.tile);
   const EnsBox& B = boxes[r.b];
   r.P = rek_to<K>(B.P);
   r.off = B.off;
-  const unsigned int local = r.tile - t0[r.b];
-  unsigned int bx, by, bz;
-  if (ZF) {
-    const unsigned int nz = (unsigned int)r.P.g.nz, rest = local / nz;
-    bz = local - rest * nz;
-    bx = rest % B.ntx;
-    by = rest / B.ntx;
-  } else {
-    const unsigned int rest = local / B.ntx;
-    bx = local - rest * B.ntx;
-    by = rest % B.nty;
-    bz = rest / B.nty;
-  }
-  r.t = cell_at(r.P.g, bx, by, bz);
+  const unsigned int local = r.tile - t0[r.b], n = ZF ? (unsigned int)r.P.g.nz : (unsigned int)B.ncol;
+  const unsigned int slow = local / n, fast = local - slow * n;
+  r.t.k = (int)(ZF ? fast : slow);
+  r.t.valid = tile_column(B, ZF ? slow : fast, r.t.i, r.t.j);
+  r.t.c = r.t.valid ? r.P.g.idx(r.t.i, r.t.j, r.t.k) : 0;
   return r;
 }
 
@@ -111,91 +97,72 @@ struct BoxCol {
   bool valid;
 };
 
+__device__ __forceinline__ void box_col_at(const EnsBox& B, unsigned int local, BoxCol& r) {
+  const unsigned int bz = local / (unsigned int)B.ncol, col = local - bz * (unsigned int)B.ncol;
+  r.off = B.off;
+  r.g = B.P.g;
+  r.valid = tile_column(B, col, r.i, r.j);
+  r.k0 = (int)bz * B.kc;
+  r.k1 = min(r.g.nz, r.k0 + B.kc);
+}
+
 __device__ __forceinline__ BoxCol box_col(const EnsBox* boxes, const unsigned int* s0, int nbox) {
   BoxCol r;
   r.tile = xcd_remap(blockIdx.x, gridDim.x);
   r.b = find_box(s0, nbox, r.tile);
-  const EnsBox& B = boxes[r.b];
-  r.off = B.off;
-  r.g = B.P.g;
-  const unsigned int local = r.tile - s0[r.b];
-  const unsigned int bx = local % B.ntx, rest = local / B.ntx, by = rest % B.nty, bz = rest / B.nty;
-  r.i = bx * 64 + (threadIdx.x & 63);
-  r.j = by * 4 + (threadIdx.x >> 6);
-  r.k0 = bz * B.kc;
-  r.k1 = min(r.g.nz, r.k0 + B.kc);
-  r.valid = r.i < r.g.nx && r.j < r.g.ny;
+  box_col_at(boxes[r.b], r.tile - s0[r.b], r);
   return r;
 }
 
 // ---- Richards kernels ------------------------------------------------------------------------
 
-__global__ __launch_bounds__(NT) void kb_save(const EnsBox* boxes, const unsigned int* t0, int nbox, Pools F) {
-  const BoxCell q = box_cell(boxes, t0, nbox);
-  if (!q.t.valid) return;
-  const long long c = q.off + q.t.c;
-  F.hn[c] = F.h[c];
-  F.wcn[c] = F.wc[c];
-}
-
-// Ghost cells of h^n / theta^n: the face ghosts of every boundary cell (corner ghosts are unused).
-__global__ __launch_bounds__(NT) void kb_save_ghosts(const EnsBox* boxes, const unsigned int* t0, int nbox, Pools F) {
-  const BoxCell q = box_cell(boxes, t0, nbox);
+// Start of a step: h^n and theta^n (with their ghost cells), K and C at h^n, and x0 on interior cells by
+// `mode`: 0 zero, 1 h^n, 2 (extrapolated start) h^n plus the increment of the last step's solve, in the
+// single-box arithmetic (k_extrap_interior); hn still holds that step's starting head, hp its
+// post-solve head. Each cell writes the ghost cells that it faces, which only it reads here.
+// One pass instead of four (save, ghosts, K and C, start): of the 96 bytes per cell that they moved,
+// 72 are left.
+template <class K, int ZF>
+__global__ __launch_bounds__(NT) void kb_start(const EnsBox* boxes, const unsigned int* t0, int nbox, Pools F,
+                                               int mode) {
+  const BoxCell<K> q = box_cell<K, ZF>(boxes, t0, nbox);
   if (!q.t.valid) return;
   const Geo& g = q.P.g;
   const Cell& t = q.t;
+  double* h = F.h + q.off;
+  double* hn = F.hn + q.off;
+  const double* wc = F.wc + q.off;
+  double* wcn = F.wcn + q.off;
+  const double hc = h[t.c];
+  if (mode == 2) h[t.c] = hc + (F.hp[q.off + t.c] - hn[t.c]);
+  if (mode == 0) h[t.c] = 0.0;
+  hn[t.c] = hc;
+  wcn[t.c] = wc[t.c];
   const long long gh[6] = {t.i == 0 ? t.c - 1 : -1,    t.i == g.nx - 1 ? t.c + 1 : -1,
                            t.j == 0 ? t.c - g.sy : -1, t.j == g.ny - 1 ? t.c + g.sy : -1,
                            t.k == 0 ? t.c - g.sz : -1, t.k == g.nz - 1 ? t.c + g.sz : -1};
 #pragma unroll
-  for (int k = 0; k < 6; ++k)
-    if (gh[k] >= 0) {
-      F.hn[q.off + gh[k]] = F.h[q.off + gh[k]];
-      F.wcn[q.off + gh[k]] = F.wc[q.off + gh[k]];
+  for (int f = 0; f < 6; ++f)
+    if (gh[f] >= 0) {
+      hn[gh[f]] = h[gh[f]];
+      wcn[gh[f]] = wc[gh[f]];
     }
-}
-
-template <class K, int ZF>
-__global__ __launch_bounds__(NT) void kb_pre(const EnsBox* boxes, const unsigned int* t0, int nbox, Pools F) {
-  const BoxCellT<K> q = box_cell_as<K, ZF>(boxes, t0, nbox);
-  if (q.t.valid) re_pre(q.P, q.t, F.hn + q.off, F.kr + q.off, F.ch + q.off);
+  re_pre(q.P, t, hn, F.kr + q.off, F.ch + q.off);
 }
 
 template <class K, int ZF>
 __global__ __launch_bounds__(NT) void kb_assemble(const EnsBox* boxes, const unsigned int* t0, int nbox, Pools F,
                                                    float* D32, float* ax32, float* ay32, float* az32) {
-  const BoxCellT<K> q = box_cell_as<K, ZF>(boxes, t0, nbox);
+  const BoxCell<K> q = box_cell<K, ZF>(boxes, t0, nbox);
   if (!q.t.valid) return;
   const long long o = q.off;
   re_assemble(q.P, q.t, F.kr + o, F.ch + o, F.wcn + o, F.hn + o, F.D + o, F.ax + o, F.ay + o, F.az + o, F.rhs + o,
               D32 ? D32 + o : nullptr, ax32 + o, ay32 + o, az32 + o);
 }
 
-// kb_save for the extrapolated start with a previous increment: before h^n is overwritten (it
-// still holds the last step's starting head), the start h^n + (post-solve head - that head) goes
-// to hp, in the single-box arithmetic (k_extrap_interior).
-__global__ __launch_bounds__(NT) void kb_save_extrap(const EnsBox* boxes, const unsigned int* t0, int nbox, Pools F) {
-  const BoxCell q = box_cell(boxes, t0, nbox);
-  if (!q.t.valid) return;
-  const long long c = q.off + q.t.c;
-  const double h = F.h[c];
-  F.hp[c] = h + (F.hp[c] - F.hn[c]);
-  F.hn[c] = h;
-  F.wcn[c] = F.wc[c];
-}
-
-// x0 on interior cells: 0 (mode 0), h^n (1), or the extrapolated start kept in hp (2).
-__global__ __launch_bounds__(NT) void kb_guess(const EnsBox* boxes, const unsigned int* t0, int nbox, Pools F,
-                                                int mode) {
-  const BoxCell q = box_cell(boxes, t0, nbox);
-  if (!q.t.valid) return;
-  const long long c = q.off + q.t.c;
-  F.h[c] = mode == 2 ? F.hp[c] : (mode == 1 ? F.hn[c] : 0.0);
-}
-
 template <class K, int ZF>
 __global__ __launch_bounds__(NT) void kb_post(const EnsBox* boxes, const unsigned int* t0, int nbox, Pools F) {
-  const BoxCellT<K> q = box_cell_as<K, ZF>(boxes, t0, nbox);
+  const BoxCell<K> q = box_cell<K, ZF>(boxes, t0, nbox);
   if (!q.t.valid) return;
   if (F.hp) F.hp[q.off + q.t.c] = F.h[q.off + q.t.c];  // the post-solve head (extrapolated start)
   re_post(q.P, q.t, F.h + q.off, F.kr + q.off, F.ch + q.off, F.wch + q.off);
@@ -207,7 +174,7 @@ __global__ __launch_bounds__(NT) void kb_flux_correct(const EnsBox* boxes, const
                                                        unsigned char* sat0, unsigned char* cand, double* part,
                                                        unsigned int ntile) {
   __shared__ double lds[NT / kWave];
-  const BoxCellT<K> q = box_cell_as<K, ZF>(boxes, t0, nbox);
+  const BoxCell<K> q = box_cell<K, ZF>(boxes, t0, nbox);
   double a = 0.0, b = 0.0, d = 0.0;
   if (q.t.valid) {
     const long long o = q.off;
@@ -229,18 +196,21 @@ __global__ void kb_clear_flags(int* flags, int n) {
   for (int i = threadIdx.x; i < n; i += blockDim.x) flags[i] = 0;
 }
 
-// Sweep s of the saturation fixed point; once a sweep changed nothing, later sweeps only copy.
-__global__ __launch_bounds__(NT) void kb_realloc(const EnsBox* boxes, const unsigned int* t0, int nbox, Pools F,
+// Sweep s of the saturation fixed point; once a sweep changed nothing, later sweeps only copy. A byte or
+// two per cell: over the SpMV tiles, whose blocks share the search for their box (70 -> 22 us).
+__global__ __launch_bounds__(NT) void kb_realloc(const EnsBox* boxes, const unsigned int* s0, int nbox, Pools F,
                                                   const unsigned char* sat0, const unsigned char* cand,
                                                   const unsigned char* prev, unsigned char* next, int* flags, int s) {
-  const BoxCell q = box_cell(boxes, t0, nbox);
-  if (!q.t.valid) return;
+  const BoxCol q = box_col(boxes, s0, nbox);
+  if (!q.valid) return;
   const long long o = q.off;
-  if (s > 0 && flags[s - 1] == 0) {
-    next[o + q.t.c] = prev[o + q.t.c];
-    return;
+  const ReK& P = boxes[q.b].P;
+  const bool settled = s > 0 && flags[s - 1] == 0;
+  Cell t{q.i, q.j, q.k0, q.g.idx(q.i, q.j, q.k0), true};
+  for (; t.k < q.k1; ++t.k, t.c += q.g.sz) {
+    if (settled) next[o + t.c] = prev[o + t.c];
+    else re_realloc(P, t, FacesK{F.Kx + o, F.Ky + o}, sat0 + o, cand + o, prev + o, next + o, flags + s);
   }
-  re_realloc(q.P, q.t, FacesK{F.Kx + o, F.Ky + o}, sat0 + o, cand + o, prev + o, next + o, flags + s);
 }
 
 template <class K, int ZF>
@@ -249,7 +219,7 @@ __global__ __launch_bounds__(NT) void kb_finalize(const EnsBox* boxes, const uns
                                                    unsigned int ntile) {
   __shared__ double lds[NT / kWave];
   __shared__ double lmax[NT / kWave];
-  const BoxCellT<K> q = box_cell_as<K, ZF>(boxes, t0, nbox);
+  const BoxCell<K> q = box_cell<K, ZF>(boxes, t0, nbox);
   double a = 0.0, b = 0.0, dh = 0.0;
   if (q.t.valid) {
     const long long o = q.off;
@@ -272,7 +242,7 @@ __global__ __launch_bounds__(NT) void kb_finalize(const EnsBox* boxes, const uns
 
 __global__ __launch_bounds__(NT) void kb_initial(const EnsBox* boxes, const unsigned int* t0, int nbox, Pools F,
                                                   int box, int from_head) {
-  const BoxCell q = box_cell(boxes, t0, nbox);
+  const BoxCell<ReK> q = box_cell<ReK, 1>(boxes, t0, nbox);
   if (q.b != box || !q.t.valid) return;
   const long long o = q.off;
   re_initial(q.P, q.t, from_head, F.h + o, F.wc + o, F.hn + o, F.wcn + o, F.wch + o, F.hwc + o, F.ch + o);
@@ -430,12 +400,11 @@ __global__ __launch_bounds__(NT) void kb_spmv(const EnsBox* boxes, const unsigne
   const EnsBox& B = boxes[b];
   const Geo g = B.P.g;
   const long long o = B.off;
-  const unsigned int local = tile - s0[b];
-  const unsigned int bx = local % B.ntx, rest = local / B.ntx, by = rest % B.nty, bz = rest / B.nty;
-  const int i = bx * 64 + (threadIdx.x & 63), j = by * 4 + (threadIdx.x >> 6);
-  const int k0 = bz * B.kc, k1 = min(g.nz, k0 + B.kc);
+  BoxCol t;
+  box_col_at(B, tile - s0[b], t);
+  const int i = t.i, j = t.j, k0 = t.k0, k1 = t.k1;
   double acc = 0.0;
-  if (i < g.nx && j < g.ny) {
+  if (t.valid) {
     const T* D = A.D + o;
     const T* ax = A.ax + o;
     const T* ay = A.ay + o;
@@ -673,12 +642,12 @@ void Ensemble::build(int nbox, const int32_t* dims, const frehg_re_params* param
     const Geo g = make_geo(nx, ny, nz);
     EnsBox& B = hbox_[b];
     B.off = storage_;
-    B.ntx = ceil_div(nx, 64);
-    B.nty = ceil_div(ny, 4);
+    B.nxp = ceil_div(nx, kRowPad) * kRowPad;
+    B.ncol = ceil_div(B.nxp * ny, NT);
     B.kc = nz;
     storage_ += g.ncell();
     cells_ += (long long)nx * ny * nz;
-    tile0_[b + 1] = tile0_[b] + (unsigned int)(B.ntx * B.nty * nz);
+    tile0_[b + 1] = tile0_[b] + (unsigned int)(B.ncol * nz);
     // default soil: the params' class, uniform
     SoilClass sc = make_soil_class(p.soil.alpha, p.soil.n, p.soil.theta_s, p.soil.theta_r, p.soil.Ks_x, p.soil.Ks_y,
                                    p.soil.Ks_z, p.soil.Ss, p.soil.use_vg, p.soil.use_mvg, p.soil.air_entry);
@@ -768,7 +737,7 @@ void Ensemble::upload_boxes() {
     if (soil_variant_code(hbox_[b].P) != variant_) variant_ = 0;
   for (int b = 0; b < nbox_; ++b) {
     const EnsBox& B = hbox_[b];
-    spmv0_[b + 1] = spmv0_[b] + (unsigned int)(B.ntx * B.nty * ceil_div(B.P.g.nz, B.kc));
+    spmv0_[b + 1] = spmv0_[b] + (unsigned int)(B.ncol * ceil_div(B.P.g.nz, B.kc));
   }
   nspmv_ = spmv0_[nbox_];
   FREHG_HIP(hipMemcpyAsync(dbox_, hbox_.data(), nbox_ * sizeof(EnsBox), hipMemcpyHostToDevice, s_));
@@ -898,18 +867,12 @@ void Ensemble::enq_prepare() {
   const EnsBox* bx = dbox_;
   const unsigned int* t0 = dtile0_;
   const int mode = prep_mode();
-  if (mode == 2)
-    hipLaunchKernelGGL(kb_save_extrap, grid, blk, 0, s_, bx, t0, nbox_, P);
-  else
-    hipLaunchKernelGGL(kb_save, grid, blk, 0, s_, bx, t0, nbox_, P);
-  hipLaunchKernelGGL(kb_save_ghosts, grid, blk, 0, s_, bx, t0, nbox_, P);
   with_soil_variant_code(variant_, [&](auto tag) {
     using K = decltype(tag);
-    hipLaunchKernelGGL((kb_pre<K, 1>), grid, blk, 0, s_, bx, t0, nbox_, P);
+    hipLaunchKernelGGL((kb_start<K, 1>), grid, blk, 0, s_, bx, t0, nbox_, P, mode);
     hipLaunchKernelGGL((kb_assemble<K, 1>), grid, blk, 0, s_, bx, t0, nbox_, P, mixed_ ? F_.D32 : nullptr, F_.ax32,
                        F_.ay32, F_.az32);
   });
-  hipLaunchKernelGGL(kb_guess, grid, blk, 0, s_, bx, t0, nbox_, P, mode);
   FREHG_LAUNCH_CHECK();
   // Krylov start: FP64 CG init, or the first refinement residual
   if (!mixed_) {
@@ -991,7 +954,7 @@ void Ensemble::enq_update(int sweeps) {
     // sweep 0 reads sat0 directly; later sweeps ping-pong between satA and satB
     const unsigned char* prev = sw == 0 ? F_.sat0 : (sw & 1 ? F_.satA : F_.satB);
     unsigned char* next = sw & 1 ? F_.satB : F_.satA;
-    hipLaunchKernelGGL(kb_realloc, grid, blk, 0, s_, bx, t0, nbox_, P, (const unsigned char*)F_.sat0,
+    hipLaunchKernelGGL(kb_realloc, dim3(nspmv_), blk, 0, s_, bx, (const unsigned int*)dspmv0_, nbox_, P, (const unsigned char*)F_.sat0,
                        (const unsigned char*)F_.cand, prev, next, flags_ + 3, sw);
   }
   FREHG_LAUNCH_CHECK();
@@ -1193,8 +1156,8 @@ void Ensemble::step(int use_graph, frehg_ens_stats* st, frehg_re_stats* per_box)
     for (; sw < kMaxSweepFlags; ++sw) {
       const unsigned char* prev = sw & 1 ? F_.satA : F_.satB;
       unsigned char* next = sw & 1 ? F_.satB : F_.satA;
-      hipLaunchKernelGGL(kb_realloc, dim3(ntile_), dim3(NT), 0, s_, (const EnsBox*)dbox_, (const unsigned int*)dtile0_,
-                         nbox_, P, (const unsigned char*)F_.sat0, (const unsigned char*)F_.cand, prev, next,
+      hipLaunchKernelGGL(kb_realloc, dim3(nspmv_), dim3(NT), 0, s_, (const EnsBox*)dbox_,
+                         (const unsigned int*)dspmv0_, nbox_, P, (const unsigned char*)F_.sat0, (const unsigned char*)F_.cand, prev, next,
                          flags_ + 3, sw);
       FREHG_LAUNCH_CHECK();
       ++extra;

@@ -19,7 +19,7 @@ namespace frehg {
 struct EnsBox {
   redev::ReK P;    // geometry, soil views and physics of the box
   long long off;   // start of the box's halo-padded storage in the field pools
-  int ntx, nty;    // 64 x 4 column tiles per layer
+  int nxp, ncol;   // lanes per row (nx padded), tiles of 256 columns per layer
   int kc;          // SpMV layers per block
   int pad;
 };
