@@ -24,9 +24,16 @@ struct EnsBox {
   int pad;
 };
 
+// Stored arrays of a box's symmetric 7-point operator (see StencilView).
+template <typename T>
+struct Sten {
+  const T *D, *ax, *ay, *az;
+};
+
 // Per-box Krylov state: outer (FP64 residual / FP64 CG) and inner (FP32 CG) control blocks.
 struct EnsCtl {
   KrylovCtl o, i;
+  int itb[2];  // CG: number of iterate `it` in itb[it & 1], as r.z in rzb
   int refinements, inner_total, parity;
   int inner_max[2];  // most inner iterations of the first refinement / of any later one
   int pad;
@@ -62,6 +69,8 @@ class Ensemble {
   void autotune();
   // Kernel sequences; each can be captured into a graph.
   void enq_prepare();                  // save h^n, theta^n; K/C; assembly; initial guess
+  template <typename T>
+  void enq_cg(const Sten<T>& A, T* x, T* r, T* z, T* p0, T* p1, T* q, int inner, int n);
   // Krylov budget (all boxes, early exit per box): FP64 iterations, or mixed refinements with
   // inner_first iterations in the first and inner_iters in each later inner solve.
   void enq_solve(int inner_iters, int refinements, int inner_first = -1);
