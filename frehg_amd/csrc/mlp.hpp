@@ -88,7 +88,7 @@ class Mlp {
   void predict_batch(const float* X, int n, float* out);
 
  private:
-  void ensure_scratch(int nrows);
+  void upload_rows(const float* X, const float* Y, int n);
   double run_grad(const float* rows, long long nrows, int batch, uint64_t seed, int sequential);
 
   hipStream_t s_;
@@ -115,8 +115,10 @@ class Mlp {
   float* grad_ = nullptr;    // reduced gradient + loss
   float* part_ = nullptr;    // per-block partial gradients
   float* log_ = nullptr;     // ring buffer, cap_ x 12
-  float* scratch_ = nullptr; // host-batch rows for the test hooks
+  float* scratch_ = nullptr; // host-batch rows for the test hooks, and their predictions
   long long scratch_rows_ = 0;
+  float* stage_ = nullptr;   // pinned: those rows on their way
+  int stage_rows_ = 0;
   double* stat_ = nullptr;   // normalisation partials
   float* hbuf_ = nullptr;    // pinned host mirror (loss)
 };
