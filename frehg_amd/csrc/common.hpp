@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cfloat>
 #include <cstdint>
 #include <stdexcept>
 #include <string>
@@ -432,7 +433,8 @@ __device__ __forceinline__ VGState vg_state(const SoilClass& s, double h) {
     const double p = fm::exp(lp);
     fm::Two l1p, d;
     if (p >= 2.5) {
-      const double e = fm::log1p_inverse(p);
+      // (of a p whose 2 p + 1 overflows, and of an infinite one, log(1 + 1/p) squared is 0)
+      const double e = p < 1e300 ? fm::log1p_inverse(p) : 0.0;
       l1p = fm::add(lp, e);
       d = fm::Two{-e, 0.0};
     } else {
@@ -440,7 +442,7 @@ __device__ __forceinline__ VGState vg_state(const SoilClass& s, double h) {
       d = fm::sub(lp, l1p);
     }
     const double sq = fm::exp(fm::mul(-0.5 * s.m, l1p));
-    se = sq * sq;
+    se = a > DBL_MAX ? 0.0 : sq * sq;  // (an infinite head: fm::log has no value for it)
     cap = s.capc * p * se / (a * (1.0 + p));
     const double t = -fm::expm1(fm::mul(s.m, d));
     kr = sq * t * t;
@@ -464,7 +466,7 @@ __device__ __forceinline__ double vg_head(const SoilClass& s, double wc) {
     if (th - s.theta_r < 1.0e-7) th = s.theta_r + 1.0e-7;
     if (th < s.theta_s) {
       const double y = fm::expm1(fm::mul(s.inv_m, fm::log((s.wcm - s.theta_r) / (th - s.theta_r))));
-      if (y == 0.0 || y > 1.7e308) return -s.inv_alpha * y;  // 0 and infinity
+      if (!(y > 0.0 && y <= DBL_MAX)) return -s.inv_alpha * (y < 0.0 ? NAN : y);  // (log y, for n < 1, has no value)
       return -s.inv_alpha * fm::exp(fm::mul(s.inv_n, fm::log(y)));
     }
     return 0.0;

@@ -76,3 +76,17 @@ def test_limits():
     assert (wch[:4] == TS).all() and (ch[:2] == 0.0).all() and (hwc[:4] == 0.0).all()
     assert np.isfinite(ch[2:5]).all() and np.isnan(wch[5]) and np.isnan(ch[5])
     assert wch[6] == pytest.approx(TR, rel=1e-12) and np.isfinite(ch[6])
+
+
+@pytest.mark.parametrize("alpha,n", CLASSES)
+def test_heads_whose_power_overflows(alpha, n):
+    """(alpha |h|)^n beyond the largest double, just below it (where twice of it overflows), and an infinite head:
+    theta is theta_r, as the closed form's limit."""
+    edge = np.exp(np.log(1.797e308) / n) / alpha  # (alpha |h|)^n = 1.797e308
+    h = -np.array([0.4 ** (1 / n) * edge, 0.7 ** (1 / n) * edge, 1.01 * edge, min(1e10 * edge, 1e300), np.inf])
+    soil = abi.soil_params(alpha=alpha, n=n, theta_s=TS, theta_r=TR, Ks_z=1e-5)
+    ctx = gpu.Context(0)
+    ctx.re_init(len(h), 1, 1, abi.re_params(soil=soil, adaptive_dt=0))
+    ctx.re_set_initial(h=h)
+    wch = ctx.re_get("wch").reshape(3, 3, len(h) + 2)[1, 1, 1:-1]
+    assert (wch == TR).all(), wch
