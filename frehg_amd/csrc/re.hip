@@ -36,6 +36,9 @@ namespace {
 using namespace redev;
 constexpr int NT = kReNT;
 
+// Whether the queued solve that this kernel runs behind has failed (stop null: nothing is outstanding).
+__device__ __forceinline__ bool stopped(const int* stop) { return stop != nullptr && *stop != 0; }
+
 // Cell of this thread; ZF selects the tile order (0: x fastest, 1: layer fastest). Layer-fastest
 // order lets the kernels with vertical stencils (assemble, flux + corrector) find the layers above
 // and below in L2; measured faster for all per-cell kernels except finalize.
@@ -76,8 +79,10 @@ __global__ __launch_bounds__(NT) void k_re_assemble(K P, const double* __restric
 }
 
 template <class K, int ZF>
-__global__ __launch_bounds__(NT) void k_re_post(K P, double* __restrict__ h, double* __restrict__ kr,
-                                                 double* __restrict__ ch, double* __restrict__ wch) {
+__global__ __launch_bounds__(NT) void k_re_post(K P, const int* __restrict__ stop, double* __restrict__ h,
+                                                 double* __restrict__ kr, double* __restrict__ ch,
+                                                 double* __restrict__ wch) {
+  if (stopped(stop)) return;
   TileId b;
   const Cell t = tile_cell<ZF>(P.g, b);
   if (t.valid) re_post(P, t, h, kr, ch, wch);
@@ -86,7 +91,8 @@ __global__ __launch_bounds__(NT) void k_re_post(K P, double* __restrict__ h, dou
 // Fluxes + corrector (re_flux_correct); ledger partials (sum theta^n V, specific-storage term,
 // boundary inflow) per block to part[0..2][nblocks].
 template <class K, int ZF>
-__global__ __launch_bounds__(NT) void k_re_flux_correct(K P, const double* __restrict__ h, const double* __restrict__ kr,
+__global__ __launch_bounds__(NT) void k_re_flux_correct(K P, const int* __restrict__ stop,
+                                                         const double* __restrict__ h, const double* __restrict__ kr,
                                                          const double* __restrict__ hn, const double* __restrict__ wcn,
                                                          const double* __restrict__ wch, double* __restrict__ Kx,
                                                          double* __restrict__ Ky, double* __restrict__ Kz,
@@ -97,6 +103,7 @@ __global__ __launch_bounds__(NT) void k_re_flux_correct(K P, const double* __res
                                                          unsigned char* __restrict__ kf, double* __restrict__ part,
                                                          unsigned int nblocks, int* __restrict__ flags, int nflags) {
   __shared__ double lds3[3 * (NT / kWave)];
+  if (stopped(stop)) return;
   TileId b;
   const Cell t = tile_cell<ZF>(P.g, b);
   if (b.linear == 0 && (int)threadIdx.x < nflags) flags[threadIdx.x] = 0;  // reallocation sweep flags
@@ -140,6 +147,7 @@ __global__ __launch_bounds__(NT) void k_re_realloc_iter(K P, FA fa, const unsign
 // theta_c) V) to part[3..4][nblocks] and max |h^{n+1} - h^n| to mx[nblocks].
 template <class K, int ZF, class FA>
 __global__ __launch_bounds__(NT) void k_re_finalize(K P, FA fa, const int* __restrict__ changed,
+                                                     const int* __restrict__ stop,
                                                      const unsigned char* __restrict__ sat0,
                                                      const unsigned char* __restrict__ fin,
                                                      const double* __restrict__ wch, const double* __restrict__ hwc,
@@ -150,6 +158,7 @@ __global__ __launch_bounds__(NT) void k_re_finalize(K P, FA fa, const int* __res
                                                      unsigned int nblocks) {
   __shared__ double lds[NT / kWave];
   __shared__ double lmax[NT / kWave];
+  if (stopped(stop)) return;
   if (changed && *changed) return;  // the sweep before changed the saturation state: not its fixed point yet
   TileId b;
   const Cell t = tile_cell<ZF>(P.g, b);
@@ -262,10 +271,11 @@ __global__ __launch_bounds__(NT) void k_re_dtadapt(ReK P, const double* qx, cons
 // cells to part[0..nblocks) (part[nblocks..) = 0 for k_reduce_maxmin), and hm = h (the iterate
 // the next test compares against; hm may be ref itself).
 template <class K, int ZF>
-__global__ __launch_bounds__(NT) void k_re_post_delta(K P, double* __restrict__ h, double* __restrict__ kr,
-                                                       double* __restrict__ ch, double* __restrict__ wch,
-                                                       const double* ref, double* hm, double* part,
-                                                       unsigned int nblocks) {
+__global__ __launch_bounds__(NT) void k_re_post_delta(K P, const int* __restrict__ stop, double* __restrict__ h,
+                                                       double* __restrict__ kr, double* __restrict__ ch,
+                                                       double* __restrict__ wch, const double* ref, double* hm,
+                                                       double* part, unsigned int nblocks) {
+  if (stopped(stop)) return;
   TileId b;
   const Cell t = tile_cell<ZF>(P.g, b);
   double d = 0.0;
@@ -393,14 +403,15 @@ __global__ __launch_bounds__(NT) void k_re_post_chunks(K P, const unsigned long 
 // on (nothing it reads is written here) and the flux kernel runs again at its last iterate.
 template <class K, int ZF>
 __global__ __launch_bounds__(NT) void k_re_check_flux_correct(
-    K P, const double* __restrict__ h, const double* __restrict__ kr, const double* __restrict__ ch,
-    const double* __restrict__ hn, const double* __restrict__ wcn, const double* __restrict__ wch,
-    double* __restrict__ Kx, double* __restrict__ Ky, double* __restrict__ Kz, double* __restrict__ qx,
+    K P, const int* __restrict__ stop, const double* __restrict__ h, const double* __restrict__ kr,
+    const double* __restrict__ ch, const double* __restrict__ hn, const double* __restrict__ wcn,
+    const double* __restrict__ wch, double* __restrict__ Kx, double* __restrict__ Ky, double* __restrict__ Kz, double* __restrict__ qx,
     double* __restrict__ qy, double* __restrict__ qz, double* __restrict__ wc, double* __restrict__ hwc,
     unsigned char* __restrict__ sat0, unsigned char* __restrict__ cand, unsigned char* __restrict__ kf,
     double* __restrict__ part, double* __restrict__ cpart, unsigned int nblocks, int* __restrict__ flags,
     int nflags) {
   __shared__ double lds5[5 * (NT / kWave)];
+  if (stopped(stop)) return;
   TileId b;
   const Cell t = tile_cell<ZF>(P.g, b);
   if (b.linear == 0 && (int)threadIdx.x < nflags) flags[threadIdx.x] = 0;  // reallocation sweep flags
@@ -488,9 +499,9 @@ __global__ __launch_bounds__(NT) void k_re_initial(ReK P, int from_head, double*
 }
 
 // x0 = h^n on interior cells (previous-step initial guess).
-__global__ __launch_bounds__(NT) void k_copy_interior(Geo g, const double* src, double* dst) {
+__global__ __launch_bounds__(NT) void k_copy_interior(Geo g, const int* stop, const double* src, double* dst) {
   const Cell t = cell_of(g);
-  if (!t.valid) return;
+  if (!t.valid || stopped(stop)) return;
   dst[t.c] = src[t.c];
 }
 
@@ -864,7 +875,7 @@ void ReState::step(frehg_re_stats* st) {
   bool post0 = false;  // the start kernels took the post-solve pass at h^0
   const long long nchunks = (long long)ceil_div(g_.nx, 64) * g_.ny * g_.nz;  // 64-cell row chunks
   if (p_.initial_guess == FREHG_GUESS_PREVIOUS || (p_.initial_guess == FREHG_GUESS_EXTRAPOLATED && !have_inc)) {
-    hipLaunchKernelGGL(k_copy_interior, grid, blk, 0, s_, g_, hn_, h_);
+    hipLaunchKernelGGL(k_copy_interior, grid, blk, 0, s_, g_, nullptr, hn_, h_);
     FREHG_LAUNCH_CHECK();
     x0_zero = false;
   } else if (p_.initial_guess == FREHG_GUESS_EXTRAPOLATED) {
@@ -941,8 +952,8 @@ void ReState::step(frehg_re_stats* st) {
       with_soil_variant(P, [&](const auto& PK) {
         using K = std::decay_t<decltype(PK)>;
         // post-solve pass at h^0, which also keeps h^0 in hp_ (its test output is not used)
-        hipLaunchKernelGGL((k_re_post_delta<K, 1>), grid, blk, 0, s_, PK, h_, kr_, ch_, wch_, (const double*)hn_,
-                           hp_, red_, nbl);
+        hipLaunchKernelGGL((k_re_post_delta<K, 1>), grid, blk, 0, s_, PK, nullptr, h_, kr_, ch_, wch_,
+                           (const double*)hn_, hp_, red_, nbl);
         FREHG_LAUNCH_CHECK();
       });
     swept = assemble(mixed, true);
@@ -993,6 +1004,9 @@ void ReState::step(frehg_re_stats* st) {
   local.guess_fallback = sr.guess_rejected ? 1 : 0;
   local.picard_iterations = 1;
   local.picard_converged = p_.picard_max > 1 ? 0 : 1;
+  // The kernels queued behind a solve whose outcome the host has not seen leave the state alone when it has
+  // failed: an error then leaves the step's fields as it does when the host waits for the solve.
+  auto stop = [&]() -> const int* { return queued ? kry_->failed_flag() : nullptr; };
   // Once the stream has drained: the outcome of a queued solve. When it has to be solved again (true), the
   // work queued behind it has to be queued again too.
   auto resolve = [&](bool zero, bool first) -> bool {
@@ -1016,7 +1030,8 @@ void ReState::step(frehg_re_stats* st) {
     const bool zero = p_.initial_guess == FREHG_GUESS_ZERO;
     with_soil_variant(P, [&](const auto& PK) {
       using K = std::decay_t<decltype(PK)>;
-      hipLaunchKernelGGL((k_re_post_delta<K, 1>), grid, blk, 0, s_, PK, h_, kr_, ch_, wch_, ref, hp_, red_, nbl);
+      hipLaunchKernelGGL((k_re_post_delta<K, 1>), grid, blk, 0, s_, PK, stop(), h_, kr_, ch_, wch_, ref, hp_, red_,
+                         nbl);
       FREHG_LAUNCH_CHECK();
     });
     post_done = true;
@@ -1043,7 +1058,7 @@ void ReState::step(frehg_re_stats* st) {
       with_soil_variant(P, [&](const auto& PK) {
         using K = std::decay_t<decltype(PK)>;
         if (check_flux_)
-          hipExtLaunchKernelGGL((k_re_check_flux_correct<K, 1>), grid, blk, 0, s_, ev0, ev1, 0, PK,
+          hipExtLaunchKernelGGL((k_re_check_flux_correct<K, 1>), grid, blk, 0, s_, ev0, ev1, 0, PK, stop(),
                                 (const double*)h_, (const double*)kr_, (const double*)ch_, (const double*)hn_,
                                 (const double*)wcn_, (const double*)wch_, Kx_, Ky_, Kz_, qx_, qy_, qz_, wc_, hwc_,
                                 sat0_, cand_, lazy_flux_ ? kf_ : nullptr, led_, red_, nbl, dflag_, kSweepFlags);
@@ -1057,17 +1072,11 @@ void ReState::step(frehg_re_stats* st) {
     }
     // hres_ (written by the reductions): [0] the Picard test's max |dh|, [11..12] the residual test's sums
     FREHG_HIP(hipStreamSynchronize(s_));
-    // (a solve that had to be done again invalidates what was queued behind it: the loop goes on)
-    const bool again = resolve(m == 1 ? x0_zero : zero, m == 1);
-    if (again) {
-      with_soil_variant(P, [&](const auto& PK) {
-        using K = std::decay_t<decltype(PK)>;
-        hipLaunchKernelGGL((k_re_post_delta<K, 1>), grid, blk, 0, s_, PK, h_, kr_, ch_, wch_, (const double*)hp_,
-                           hp_, red_, nbl);
-        FREHG_LAUNCH_CHECK();
-      });
+    if (resolve(m == 1 ? x0_zero : zero, m == 1)) {  // solved again: the passes at h^m now
+      --m;
+      continue;
     }
-    if (m > 1 && !zero && unchanged && !again) {
+    if (m > 1 && !zero && unchanged && hres_[0] == 0.0) {
       // a solve from h^{m-1} that returned it unchanged ended the loop before this iterate in the waiting form;
       // here the passes at h^m = h^{m-1} have repeated their results
       local.picard_converged = 1;
@@ -1075,13 +1084,13 @@ void ReState::step(frehg_re_stats* st) {
       skip_check_ &= ~(m - 1 < 32 ? 1u << (m - 1) : 0u);
       break;
     }
-    if (!again && hres_[0] <= p_.picard_tol) {
+    if (hres_[0] <= p_.picard_tol) {
       local.picard_converged = 1;
       flux_done = spec && check_flux_;
       break;
     }
     if (m >= p_.picard_max) break;  // the cap: the step continues from the last iterate
-    if (spec && !again) {
+    if (spec) {
       const double rr = hres_[11], bb = hres_[12];
       const double ttol = std::fmax(kc.rtol * std::sqrt(bb), kc.atol);
       if (rr <= ttol * ttol) {
@@ -1160,11 +1169,11 @@ void ReState::step(frehg_re_stats* st) {
     with_soil_variant(P, [&](const auto& PK) {
       using K = std::decay_t<decltype(PK)>;
       if (lazy_flux_)
-        hipLaunchKernelGGL((k_re_finalize<K, 0, FacesF>), grid, blk, 0, s_, PK, FacesF{kf_}, changed,
+        hipLaunchKernelGGL((k_re_finalize<K, 0, FacesF>), grid, blk, 0, s_, PK, FacesF{kf_}, changed, stop(),
                            (const unsigned char*)sat0_, prev, (const double*)wch_, (const double*)hwc_,
                            (const double*)hn_, wc_, h_, hp_, hmod_, led_, led_ + 5 * (size_t)nbl, nbl);
       else
-        hipLaunchKernelGGL((k_re_finalize<K, 0, FacesK>), grid, blk, 0, s_, PK, FacesK{Kx_, Ky_}, changed,
+        hipLaunchKernelGGL((k_re_finalize<K, 0, FacesK>), grid, blk, 0, s_, PK, FacesK{Kx_, Ky_}, changed, stop(),
                            (const unsigned char*)sat0_, prev, (const double*)wch_, (const double*)hwc_,
                            (const double*)hn_, wc_, h_, nullptr, hmod_, led_, led_ + 5 * (size_t)nbl, nbl);
       FREHG_LAUNCH_CHECK();
@@ -1177,7 +1186,7 @@ void ReState::step(frehg_re_stats* st) {
     // Without lazy fluxes finalize writes the final head over the post-solve head: keep the latter
     // in hp_ for the next step's increment.
     if (track_inc && !lazy_flux_) {
-      hipLaunchKernelGGL(k_copy_interior, grid, blk, 0, s_, g_, (const double*)h_, hp_);
+      hipLaunchKernelGGL(k_copy_interior, grid, blk, 0, s_, g_, stop(), (const double*)h_, hp_);
       FREHG_LAUNCH_CHECK();
     }
     if (!flux_done) {
@@ -1186,11 +1195,11 @@ void ReState::step(frehg_re_stats* st) {
       with_soil_variant(P, [&](const auto& PK) {
         using K = std::decay_t<decltype(PK)>;
         if (!post_done) {
-          hipExtLaunchKernelGGL((k_re_post<K, 1>), grid, blk, 0, s_, ev0, nullptr, 0, PK, h_, kr_, ch_, wch_);
+          hipExtLaunchKernelGGL((k_re_post<K, 1>), grid, blk, 0, s_, ev0, nullptr, 0, PK, stop(), h_, kr_, ch_, wch_);
           FREHG_LAUNCH_CHECK();
         }
         hipExtLaunchKernelGGL((k_re_flux_correct<K, 1>), grid, blk, 0, s_, post_done ? ev0 : nullptr, ev1, 0, PK,
-                              (const double*)h_, (const double*)kr_, (const double*)hn_, (const double*)wcn_,
+                              stop(), (const double*)h_, (const double*)kr_, (const double*)hn_, (const double*)wcn_,
                               (const double*)wch_, Kx_, Ky_, Kz_, qx_, qy_, qz_, wc_, hwc_, sat0_, cand_,
                               lazy_flux_ ? kf_ : nullptr, led_, nbl, dflag_, kSweepFlags);
         FREHG_LAUNCH_CHECK();
