@@ -532,7 +532,8 @@ int frehg_ls_solve_noalloc(frehg_ctx_t ctx, int ndim, int nx, int ny, int nz, co
                            const frehg_solver_config* cfg, frehg_solve_stats* st) {
   return guard(ctx, [&] {
     if (!cfg) throw frehg::ArgError("frehg_ls_solve_noalloc: null argument");
-    frehg::ls_solve_noalloc(ctx->device, ctx->stream, ndim, nx, ny, nz, diag, offdiag, b_owned, x_owned, *cfg, st);
+    frehg::ls_solve_noalloc(ctx->device, ctx->stream, ndim, nx, ny, nz, diag, offdiag, b_owned, x_owned, *cfg, st,
+                            &ctx->prof.resident);
     return FREHG_OK;
   });
 }
@@ -578,6 +579,17 @@ int frehg_spmv_shape(frehg_ctx_t ctx, int precision, int* cells_per_lane, int* k
     const frehg::Krylov::SpmvShape& sh = re.krylov().spmv_shape(precision == FREHG_PREC_MIXED ? 1 : 0);
     if (cells_per_lane) *cells_per_lane = sh.cpl;
     if (kchunk) *kchunk = sh.kc;
+    return FREHG_OK;
+  });
+}
+
+int frehg_resident_use(frehg_ctx_t ctx, int64_t* launches, int64_t* gave_up, int* cells_per_thread, int* blocks) {
+  return guard(ctx, [&] {
+    const frehg::ResidentUse& u = ctx->prof.resident;
+    if (launches) *launches = u.launches;
+    if (gave_up) *gave_up = u.gave_up;
+    if (cells_per_thread) *cells_per_thread = u.cells_per_thread;
+    if (blocks) *blocks = u.blocks;
     return FREHG_OK;
   });
 }

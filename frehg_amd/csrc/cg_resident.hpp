@@ -25,9 +25,15 @@
 // exchange k + 2 only after it has seen every block's sums of exchange k + 1, which each block posts after its
 // last look at the words of exchange k.
 //
-// The grid is at most one block per compute unit, so all blocks are resident together. Should a block
-// be kept from starting (another process's kernel of this kind on the same device), the waits end after
-// kCgWaitTicks, the launch reports a time-out, and the caller solves with the streaming kernels.
+// The grid is at most one block per compute unit (a compute unit holds one: 512 threads of up to 252 registers),
+// so all blocks of a launch that has the device to itself are resident together. Another process's launches of this
+// kind, or any kernel that holds compute units, can keep some of them from starting, and two such launches that
+// hold a part of the device each would wait for one another. So a block reports at its gate as it starts and, once
+// its part of the operator is loaded, looks whether all have; it closes the gate of a block that has not
+// reported within kCgGateTicks. A gate is either passed or closed for good, so all blocks see the same and with
+// a closed one all leave, x as it was. Behind the gates every block is on the device and the waits are short; a
+// bound on them (kCgWaitTicks and kCgWaitLooks) is left so that they end whatever happens. Either way the
+// launch reports that it gave up, and the caller solves with the streaming kernels.
 #pragma once
 
 #include <type_traits>
@@ -41,9 +47,12 @@ constexpr int kCgNT = 512;          // threads per block
 constexpr int kCgHalo = 4;          // halo cells per thread, at most
 constexpr int kCgMailWords = 10;    // 8-byte words that one block posts per exchange
 constexpr int kCgMaxBlocks = 512;   // one polling thread per block
-constexpr int kCgMaxLds = 62 * 1024;        // dynamic LDS with the operator in registers (two blocks fit a CU)
+constexpr int kCgMailFront = kCgMaxBlocks / 2;  // words before the posted ones: the gates, 32 bits per block
+constexpr int kCgMaxLds = 62 * 1024;        // dynamic LDS with the operator in registers
 constexpr int kCgMaxLdsOp = 158 * 1024;     // and with the operator in LDS (the rest is for the reductions)
-constexpr long long kCgWaitTicks = 25000000;  // 0.25 s of the 100 MHz wall clock
+// Looks before kCgWaitTicks may end a wait (tens of milliseconds): the clock also runs while the device has
+// switched the waves out for another process's.
+constexpr unsigned int kCgWaitLooks = 1u << 16;
 
 template <typename T>
 struct CgResidentArgs {
@@ -56,14 +65,16 @@ struct CgResidentArgs {
   const T* r0;               // started by a refinement sweep: its residual (b, bn unused, x0 = 0)
   const KrylovCtl* ctl;      // and its control block
   KrylovCtl* out;            // result (device or pinned host memory)
-  int* timeout;              // set to 1 when a wait ends without its word
+  int* gave_up;              // set to 1 when a wait ends without its word
   int* failed;               // device word for kernels queued behind: set to 1 unless the solve converges
   double rtol, atol;
   int max_it, guard, x0_zero;
   int tx, ty, tz, ntx, nty, ntz;  // cells per tile, tiles
   unsigned long long *lo[2], *hi[2];  // a tagged word per cell and half (hi: FP64 only)
-  unsigned long long* mail;           // 2 x kCgMailWords x blocks
-  unsigned int launch;       // 1 .. 2^20 - 1
+  unsigned long long* mail;  // 2 x kCgMailWords x blocks, the gates before them
+  unsigned int launch;       // 1 .. 2^19 - 1
+  // see kCgGateTicks; for tests of the recovery, 0: block 0 closes its own gate / leaves after the first iteration
+  long long gate_ticks, wait_ticks;
 };
 
 __device__ __forceinline__ void cg_put(unsigned long long* p, unsigned long long v) {
@@ -75,8 +86,29 @@ __device__ __forceinline__ unsigned long long cg_get(const unsigned long long* p
 __device__ __forceinline__ void cg_fail(int* failed) {
   __hip_atomic_store(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void cg_give_up(int* gave_up, int* failed) {
+  __hip_atomic_store(gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  cg_fail(failed);
+}
 __device__ __forceinline__ unsigned long long cg_tagged(unsigned int tag, unsigned int v) {
   return ((unsigned long long)tag << 32) | v;
+}
+// The gates, a 32-bit word per block before the posted words: 2 launch once the block has started, 2 launch + 1 if
+// another block closed it before that.
+__device__ __forceinline__ unsigned int* cg_gate(unsigned long long* mail, unsigned int blk) {
+  return reinterpret_cast<unsigned int*>(mail - kCgMailFront) + blk;
+}
+// Waits until block `blk` has started, or closes its gate after `ticks`; whether the gate is closed.
+__device__ __forceinline__ bool cg_closed(unsigned int* p, unsigned int launch, long long ticks) {
+  const long long t0 = wall_clock64();
+  for (;;) {
+    unsigned int was = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (was == 2 * launch || was == 2 * launch + 1) return was & 1u;
+    if (wall_clock64() - t0 > ticks &&
+        __hip_atomic_compare_exchange_strong(p, &was, 2 * launch + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT))
+      return true;
+  }
 }
 
 // Sum over a wave by DPP moves (within rows of 16, then across rows), valid in lane 63: a fixed
@@ -160,6 +192,7 @@ __global__ __launch_bounds__(kCgNT) void k_cg_resident(CgResidentArgs<T> P) {
   extern __shared__ __align__(16) unsigned char cg_lds[];
   __shared__ double red[2 * 5 * (kCgNT / kWave)];
   __shared__ int dead;
+  __shared__ long long bound;  // P.wait_ticks (looked at now and then: not worth registers)
   T* sp = reinterpret_cast<T*>(cg_lds);  // p on the tile and its halo
   const Geo& g = P.g;
   const int tid = threadIdx.x;
@@ -171,18 +204,25 @@ __global__ __launch_bounds__(kCgNT) void k_cg_resident(CgResidentArgs<T> P) {
   const int px = P.tx + 2, py = px * (P.ty + 2);
   const int ncell = P.tx * P.ty * P.tz;
   auto gidx = [&](int i, int j, int k) -> long long { return THREE_D ? g.idx(i, j, k) : g.sidx(i, j); };
+  const bool first = blk == 0 && tid == 0;
   if (P.r0 && P.ctl->done) {  // the sweep met the tolerance: the correction is zero
     for (int l = tid; l < ncell; l += kCgNT) {
       const int lx = l % P.tx, lr = l / P.tx, i = i0 + lx, j = j0 + lr % P.ty, k = k0 + lr / P.ty;
       if (i < g.nx && j < g.ny && (!THREE_D || k < g.nz)) P.x[gidx(i, j, k)] = (T)0;
     }
-    if (blk == 0 && tid == 0) {
+    if (first) {
       KrylovCtl o = *P.ctl;
       *P.out = o;
     }
     return;
   }
-  if (tid == 0) dead = 0;
+  if (tid == 0) {
+    dead = 0;
+    bound = P.wait_ticks;
+    if (nblk > 1)
+      (void)__hip_atomic_fetch_max(cg_gate(P.mail, blk), 2 * P.launch + (first && P.gate_ticks == 0 ? 1u : 0u),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   const int nsp = py * (THREE_D ? P.tz + 2 : 1);
   for (int q = tid; q < nsp; q += kCgNT) sp[q] = (T)0;
   __syncthreads();
@@ -292,6 +332,14 @@ __global__ __launch_bounds__(kCgNT) void k_cg_resident(CgResidentArgs<T> P) {
     }
   }
   __syncthreads();
+  if (nblk > 1) {
+    if (tid < (int)nblk && cg_closed(cg_gate(P.mail, tid), P.launch, P.gate_ticks)) dead = 1;
+    __syncthreads();
+    if (dead) {
+      if (tid == 0) cg_give_up(P.gave_up, P.failed);
+      return;
+    }
+  }
 
   // Pause between posting and the first look, in units of 64 clocks: a look that comes too early costs
   // more than the pause (measured, us per iteration at pauses 0 / 8 / 14 / 20 / 26 / 34: 80 thousand rows 5.9 /
@@ -368,7 +416,7 @@ __global__ __launch_bounds__(kCgNT) void k_cg_resident(CgResidentArgs<T> P) {
       if ((spin & 63u) == 63u) {
         const long long now = wall_clock64();
         if (t0 == 0) t0 = now;
-        else if (now - t0 > kCgWaitTicks) {
+        else if (now - t0 > bound && spin > (bound > 0 ? kCgWaitLooks : 0u)) {
           dead = 1;
           break;
         }
@@ -376,10 +424,7 @@ __global__ __launch_bounds__(kCgNT) void k_cg_resident(CgResidentArgs<T> P) {
     }
     cg_block_sums<N>(v, red, flip++);  // its barrier also makes `dead` visible
     if (dead) {
-      if (tid == 0) {
-        __hip_atomic_store(P.timeout, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        cg_fail(P.failed);
-      }
+      if (tid == 0) cg_give_up(P.gave_up, P.failed);
       return false;
     }
     return true;
@@ -388,6 +433,8 @@ __global__ __launch_bounds__(kCgNT) void k_cg_resident(CgResidentArgs<T> P) {
   double rz = 0.0, zz = 0.0, pq = 0.0, ttol2 = 0.0;
   int iters = 0, conv = 0, breakdown = 0, rejected = 0;
   if (P.r0) ttol2 = P.ctl->ttol2;
+  const bool leave = nblk > 1 && blk == 0 && P.wait_ticks == 0;
+  const int max_it = leave ? 1 : P.max_it;
   for (;;) {
     // q = A p, w = D^-1 q, and the sums p.q, z.q, q.w, r.z, z.z
     double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
@@ -439,7 +486,7 @@ __global__ __launch_bounds__(kCgNT) void k_cg_resident(CgResidentArgs<T> P) {
     rz = v[3];
     zz = v[4];
     conv = (zz <= ttol2) ? 1 : 0;
-    if (conv || rejected || iters >= P.max_it) break;
+    if (conv || rejected || iters >= max_it) break;
     pq = v[0];
     if (!(pq > 0.0) || !isfinite(pq)) {
       breakdown = 1;
@@ -465,12 +512,16 @@ __global__ __launch_bounds__(kCgNT) void k_cg_resident(CgResidentArgs<T> P) {
     ++iters;
     __syncthreads();
   }
+  if (leave && iters == 1) {
+    if (tid == 0) cg_give_up(P.gave_up, P.failed);
+    return;
+  }
   if (!rejected) {
 #pragma unroll
     for (int m = 0; m < CPT; ++m)
       if ((kind[m] & kVal) && !(kind[m] & kFixed)) cg_at(P.x, off[m]) = x[m];
   }
-  if (blk == 0 && tid == 0) {
+  if (first) {
     KrylovCtl o{};
     o.rz = rz;
     o.zz = zz;

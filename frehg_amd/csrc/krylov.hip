@@ -1034,7 +1034,7 @@ __global__ __launch_bounds__(NT) void k_zero_interior(Geo g, int kchunk, T* x,
 }  // namespace
 
 Krylov::Krylov(const Geo& g, bool three_d, hipStream_t stream, Profiler* prof)
-    : g_(g), three_d_(three_d), s_(stream), prof_(prof) {
+    : g_(g), three_d_(three_d), s_(stream), prof_(prof), use_(&prof->resident) {
   try {
     build();
   } catch (...) {
@@ -1043,8 +1043,9 @@ Krylov::Krylov(const Geo& g, bool three_d, hipStream_t stream, Profiler* prof)
   }
 }
 
-Krylov::Krylov(const Geo& g, bool three_d, hipStream_t stream, Profiler* prof, const KrylovWorkspace& ws)
-    : g_(g), three_d_(three_d), s_(stream), prof_(prof), borrowed_(true) {
+Krylov::Krylov(const Geo& g, bool three_d, hipStream_t stream, Profiler* prof, ResidentUse* use,
+               const KrylovWorkspace& ws)
+    : g_(g), three_d_(three_d), s_(stream), prof_(prof), use_(use), borrowed_(true) {
   setup_shapes();
   r_ = ws.r;
   z_ = ws.z;
@@ -1059,8 +1060,11 @@ Krylov::Krylov(const Geo& g, bool three_d, hipStream_t stream, Profiler* prof, c
   // the resident solve needs none of the CG vectors: its exchange buffers take their place
   double* words[4] = {r_, z_, p0_, p1_};
   for (int q = 0; q < 4; ++q) halo_[q] = reinterpret_cast<unsigned long long*>(words[q]);
-  mail_ = reinterpret_cast<unsigned long long*>(q_);
-  if (plan_[0].nblk > 1 && 2 * (size_t)plan_[0].nblk * kCgMailWords > (size_t)n_) plan_[0] = ResidentPlan{};
+  if (plan_[0].nblk > 1) {
+    mail_ = reinterpret_cast<unsigned long long*>(q_);
+    mail_words_ = kCgMailFront + 2 * (size_t)plan_[0].nblk * kCgMailWords;
+    if (mail_words_ > (size_t)n_) plan_[0] = ResidentPlan{};
+  }
   // no autotuning (it would time launches with events): two columns per lane, whole columns per
   // block in 3D, unless FREHG_SPMV_SHAPE pins a shape
   if (!tuned_[0]) {
@@ -1217,6 +1221,23 @@ void Krylov::setup_resident() {
     return;
   }
   for (int prec = 0; prec < 2; ++prec) plan_[prec] = resident_plan(g_, three_d_, prec ? 4 : 8, cus, (size_t)std::max(0, lds - 2048));
+  // FREHG_RESIDENT_WAIT="start:exchange" (microseconds): how long a launch waits for its blocks to start and, once
+  // they have, for their words. 0 gives up at once, so that tests can take the recovery.
+  if (const char* env = std::getenv("FREHG_RESIDENT_WAIT")) {
+    long long start = -1, word = -1;
+    if (std::sscanf(env, "%lld:%lld", &start, &word) != 2 || start < 0 || word < 0 || start > 1000000 || word > 1000000)
+      throw ArgError(std::string("FREHG_RESIDENT_WAIT must be \"start:exchange\" in microseconds (0 to 1000000), got \"") +
+                     env + "\"");
+    gate_ticks_ = 100 * start;
+    wait_ticks_ = 100 * word;
+  }
+}
+
+bool Krylov::resident_turn(int prec) {
+  if (plan_[prec].cpt == 0) return false;
+  if (plan_[prec].nblk == 1 || use_->skip == 0) return true;
+  --use_->skip;
+  return false;
 }
 
 void Krylov::clear_exchange() {
@@ -1238,7 +1259,7 @@ void Krylov::build() {
   FREHG_HIP(hipHostMalloc(&host_ctl_, 2 * sizeof(KrylovCtl), hipHostMallocDefault));
   const unsigned int nblk = std::max(plan_[0].nblk, plan_[1].nblk);
   if (nblk > 1) {
-    mail_words_ = 2 * (size_t)nblk * kCgMailWords;
+    mail_words_ = kCgMailFront + 2 * (size_t)nblk * kCgMailWords;
     for (unsigned long long*& h : halo_) FREHG_HIP(hipMalloc(&h, (size_t)n_ * sizeof(unsigned long long)));
     FREHG_HIP(hipMalloc(&mail_, mail_words_ * sizeof(unsigned long long)));
     clear_exchange();
@@ -1513,9 +1534,9 @@ void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T
                              bool zero, bool guard, double rtol, double atol, int max_it, const T* r0,
                              const KrylovCtl* started) {
   const ResidentPlan& pl = plan_[sizeof(T) == 4 ? 1 : 0];
-  if (++launch_ >= (1u << 20)) {  // the tags start again: no old one may be left
+  if (++launch_ >= (1u << 19)) {  // the tags start again: no old one may be left
     launch_ = 1;
-    if (mail_words_) clear_exchange();
+    if (mail_) clear_exchange();
   }
   CgResidentArgs<T> a;
   a.g = g_;
@@ -1530,7 +1551,7 @@ void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T
   KrylovCtl* out = host_out_ ? host_ctl_ : ctl_;
   host_ctl_[1].iters = 0;
   a.out = out;
-  a.timeout = &out[1].iters;
+  a.gave_up = &out[1].iters;
   a.failed = failed_flag();
   if (failed_dirty_ && !borrowed_) FREHG_HIP(hipMemsetAsync(a.failed, 0, sizeof(int), s_));  // (borrowed: cleared)
   failed_dirty_ = true;  // until its outcome has been seen
@@ -1549,7 +1570,9 @@ void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T
     a.lo[h] = halo_[h];
     a.hi[h] = halo_[2 + h];
   }
-  a.mail = mail_;
+  a.mail = mail_ ? mail_ + kCgMailFront : nullptr;
+  a.gate_ticks = gate_ticks_;
+  a.wait_ticks = wait_ticks_;
   a.launch = launch_;
   std::unique_lock<std::mutex> lock;
   if (pl.nblk > 1) {
@@ -1559,16 +1582,26 @@ void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T
     turn.last = s_;
     turn.owner = this;
   }
+  multi_ = pl.nblk > 1;
+  use_->launches += 1;
+  use_->cells_per_thread = pl.cpt;
+  use_->blocks = (int)pl.nblk;
   if (three_d_) launch_resident<T, true>(pl.cpt, pl.nblk, pl.lds, s_, a);
   else launch_resident<T, false>(pl.cpt, pl.nblk, pl.lds, s_, a);
 }
 
+// A launch that gave up found the device shared: the next one of the context is tried after as many streamed
+// solves as the last time twice, up to 64, so that waiting in vain (5 ms) stays a small part of the time, and a
+// device that is free again is used again.
 bool Krylov::resident_ended() {
   if (host_ctl_[1].iters == 0) {
     failed_dirty_ = !host_ctl_->converged;
+    if (multi_) use_->pause = 0;
     return true;
   }
-  plan_[0] = plan_[1] = ResidentPlan{};
+  use_->gave_up += 1;
+  use_->pause = std::min(64, std::max(1, 2 * use_->pause));
+  use_->skip = use_->pause;
   return false;
 }
 
@@ -1592,13 +1625,16 @@ bool Krylov::cg_resident(const StencilView<T>& A, const T* b, const T* bn, T* x,
 
 bool Krylov::enqueue(const StencilView<double>& A, const double* b, const double* bn, double* x,
                      const unsigned char* fixed, bool x0_zero, const KrylovConfig& cfg) {
-  if (cfg.ksp != FREHG_KSP_CG || cfg.precision != 0 || !host_out_ || !resident(0) || !A.symmetric()) return false;
+  if (cfg.ksp != FREHG_KSP_CG || cfg.precision != 0 || !host_out_ || !resident(0) || !A.symmetric()) return false;  // (solve() counts a skipped turn)
   resident_launch<double>(A, b, bn, x, fixed, x0_zero, false, cfg.rtol, cfg.atol, cfg.max_it, nullptr, nullptr);
   return true;
 }
 
 bool Krylov::finish_queued(SolveResult* res) {
-  if (!resident_ended()) return false;
+  if (!resident_ended()) {
+    use_->skip += 1;  // (the caller's solve() counts a turn that is this solve's own)
+    return false;
+  }
   bool conv = false;
   *res = SolveResult{};
   res->iterations = cg_outcome<double>(&res->residual_norm, &res->rhs_norm, &conv);
@@ -1619,7 +1655,7 @@ int Krylov::run_pcg(const StencilView<T>& A, const T* b, const T* bn, T* x, cons
                     T* r, T* z, T* p0, T* p1, T* q, bool* rejected, double* res_norm,
                     double* rhs_norm, bool* converged, int kt_spmv) {
   *rejected = false;
-  if (resident(sizeof(T) == 4 ? 1 : 0)) {
+  if (resident_turn(sizeof(T) == 4 ? 1 : 0)) {
     bool ok = cg_resident<T>(A, b, bn, x, fixed, x0_zero, guard, rtol, atol, max_it, nullptr, nullptr);
     if (ok && host_ctl_->guess_rejected) {
       *rejected = true;
@@ -1883,7 +1919,7 @@ SolveResult Krylov::solve(const StencilView<double>& A, const StencilView<float>
     const double inner_rt = std::min(0.5, std::max(cfg.inner_rtol, 0.5 * gap));
     if (fused) {
       // started by the sweep (same tolerance, computed on the device)
-      if (resident(1) && cg_resident<float>(A32v, nullptr, nullptr, d32_, nullptr, true, false, 0.0, 0.0, cfg.max_it,
+      if (resident_turn(1) && cg_resident<float>(A32v, nullptr, nullptr, d32_, nullptr, true, false, 0.0, 0.0, cfg.max_it,
                                             r32_, inner)) {
         res.iterations += cg_outcome<float>(&rn, &bnrm, &iconv);
       } else {

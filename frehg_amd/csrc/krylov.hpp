@@ -56,6 +56,12 @@ struct KrylovWorkspace {
   long long n = 0;
 };
 
+// Bounds of the waits inside a resident launch (cg_resident.hpp), in ticks of the 100 MHz wall clock: for its
+// blocks to start, 5 ms (a launch that waits longer than some solves of the streaming kernels take has
+// lost), and for the words of blocks that have started, 0.25 s.
+constexpr long long kCgGateTicks = 500000;
+constexpr long long kCgWaitTicks = 25000000;
+
 struct SolveResult {
   int iterations = 0;
   int refinements = 0;
@@ -91,7 +97,7 @@ class Krylov {
   // A solver that allocates nothing: FP64 CG only, on the caller's workspace (which it does not
   // free), with a fixed SpMV shape instead of the autotuner. Its work vectors must hold finite
   // values (the SpMV meets their ghost entries with zero coefficients).
-  Krylov(const Geo& g, bool three_d, hipStream_t stream, Profiler* prof, const KrylovWorkspace& ws);
+  Krylov(const Geo& g, bool three_d, hipStream_t stream, Profiler* prof, ResidentUse* use, const KrylovWorkspace& ws);
   ~Krylov();
   // Device bytes of a borrowed workspace for this geometry, and its layout at `base` (256-byte
   // aligned pieces).
@@ -157,7 +163,8 @@ class Krylov {
     size_t lds = 0;
   };
   static ResidentPlan resident_plan(const Geo& g, bool three_d, size_t elt, int max_blocks, size_t max_lds);
-  bool resident(int prec) const { return plan_[prec].cpt > 0; }
+  // Whether the next CG solve of this precision is tried as one launch (see resident_ended for the pause).
+  bool resident(int prec) const { return plan_[prec].cpt > 0 && (plan_[prec].nblk == 1 || use_->skip == 0); }
   unsigned int resident_blocks(int prec) const { return plan_[prec].nblk; }  // 0: the solve streams
 
  private:
@@ -165,11 +172,12 @@ class Krylov {
   void clear_exchange();
   // One launch of the resident kernel (r0 / started: a solve begun by a refinement sweep, x0 = 0); once the
   // stream has drained its outcome is in host_ctl_ and resident_ended() is false when a wait inside the
-  // launch ran out (x may hold a mixture of iterates; the instance then streams).
+  // launch ran out (x may hold a mixture of iterates; the caller solves with the streaming kernels).
   template <typename T>
   void resident_launch(const StencilView<T>& A, const T* b, const T* bn, T* x, const unsigned char* fixed, bool zero,
                        bool guard, double rtol, double atol, int max_it, const T* r0, const KrylovCtl* started);
   bool resident_ended();
+  bool resident_turn(int prec);  // resident(), counting a skipped turn
   void resident_leave();
   // The launch, and the wait for it.
   template <typename T>
@@ -220,6 +228,7 @@ class Krylov {
   bool three_d_;
   hipStream_t s_;
   Profiler* prof_;
+  ResidentUse* use_;  // of the context
   SpmvShape shape_[2];
   int kc_f_ = 1;
   dim3 grid_f_;
@@ -250,6 +259,8 @@ class Krylov {
   unsigned int launch_ = 0;       // resident launches of this instance (the tag of their exchanges)
   unsigned long long *halo_[4] = {}, *mail_ = nullptr;  // its exchange buffers: low, low, high, high words; sums
   size_t mail_words_ = 0;
+  long long gate_ticks_ = kCgGateTicks, wait_ticks_ = kCgWaitTicks;
+  bool multi_ = false;            // the last resident launch had several blocks
   int last_iters_ = 8;
   int last_inner_iters_ = 8;
   int last_bcg_iters_ = 8;

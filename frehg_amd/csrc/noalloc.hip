@@ -192,7 +192,7 @@ void noalloc_setup(int device) {
 
 void ls_solve_noalloc(int device, hipStream_t s, int ndim, int nx, int ny, int nz, const double* diag,
                       const double* const* offdiag, const double* b_owned, double* x_owned,
-                      const frehg_solver_config& cfg, frehg_solve_stats* st) {
+                      const frehg_solver_config& cfg, frehg_solve_stats* st, ResidentUse* use) {
   if (ndim != 2 && ndim != 3) throw ArgError("frehg_ls_solve_noalloc: ndim must be 2 or 3");
   if (nx < 1 || ny < 1 || (ndim == 3 && nz < 1)) throw ArgError("frehg_ls_solve_noalloc: bad sizes");
   if (!diag || !offdiag || !b_owned || !x_owned) throw ArgError("frehg_ls_solve_noalloc: null argument");
@@ -233,7 +233,7 @@ void ls_solve_noalloc(int device, hipStream_t s, int ndim, int nx, int ny, int n
   int* flags = &ws.host[2].iters;
   *flags = 0;
   Profiler off;  // no timing events (they would be created on first use)
-  Krylov kry(g, three, s, &off, ws);
+  Krylov kry(g, three, s, &off, use, ws);
   NaOperator op{};
   op.diag = diag;
   for (int d = 0; d < ndir; ++d) op.off[d] = offdiag[d];

@@ -5,6 +5,7 @@
 
 #include "../../include/frehg_gpu.h"
 #include "common.hpp"
+#include "profile.hpp"
 
 namespace frehg {
 
@@ -16,10 +17,10 @@ constexpr size_t kScratchBytes = (size_t)64 << 20;
 // per device, at context creation.
 void noalloc_setup(int device);
 
-// The solve itself; operator, rhs and solution are device arrays in the owned ordering. Throws
-// ArgError / HipError / ConvergenceError like the other entry points' bodies.
+// The solve itself; operator, rhs and solution are device arrays in the owned ordering; `use` is the
+// context's. Throws ArgError / HipError / ConvergenceError like the other entry points' bodies.
 void ls_solve_noalloc(int device, hipStream_t s, int ndim, int nx, int ny, int nz, const double* diag,
                       const double* const* offdiag, const double* b_owned, double* x_owned,
-                      const frehg_solver_config& cfg, frehg_solve_stats* st);
+                      const frehg_solver_config& cfg, frehg_solve_stats* st, ResidentUse* use);
 
 }  // namespace frehg

@@ -14,8 +14,18 @@ namespace frehg {
 
 constexpr int kKernelTypes = 9;  // FREHG_KT_COUNT
 
+// One context's CG solves of one launch (cg_resident.hpp): launches, those that gave up because their blocks were
+// not all on the device, and the tiling of the last one. After a launch that gave up, the next `skip` solves
+// of several blocks stream (see Krylov::resident_ended).
+struct ResidentUse {
+  long long launches = 0, gave_up = 0;
+  int cells_per_thread = 0, blocks = 0;
+  int skip = 0, pause = 0;
+};
+
 class Profiler {
  public:
+  ResidentUse resident;
   bool enabled = false;
   unsigned int mask = ~0u;  // kernel types timed while enabled (bit kt)
   hipStream_t stream = nullptr;

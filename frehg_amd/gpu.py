@@ -76,6 +76,7 @@ def load():
         "frehg_profile_read": (C.c_int, [ctx, C.c_int, dp, P(C.c_int64)]),
         "frehg_profile_reset": (C.c_int, [ctx]),
         "frehg_spmv_shape": (C.c_int, [ctx, C.c_int, P(C.c_int), P(C.c_int)]),
+        "frehg_resident_use": (C.c_int, [ctx, P(C.c_int64), P(C.c_int64), P(C.c_int), P(C.c_int)]),
         "frehg_ens_init": (C.c_int, [ctx, C.c_int, P(C.c_int32), P(abi.ReParams)]),
         "frehg_ens_set_soil": (C.c_int, [ctx, C.c_int, P(abi.SoilParams), C.c_int, P(C.c_int32), C.c_int, dp]),
         "frehg_ens_set_initial": (C.c_int, [ctx, C.c_int, dp, dp]),
@@ -523,6 +524,12 @@ class Context:
         ty, kc = C.c_int(), C.c_int()
         self.check(self.lib.frehg_spmv_shape(self.h, precision, C.byref(ty), C.byref(kc)))
         return ty.value, kc.value
+
+    def resident_use(self):
+        """frehg_resident_use: (launches, launches that gave up, cells per thread and blocks of the last)."""
+        n, g, c, b = C.c_int64(), C.c_int64(), C.c_int(), C.c_int()
+        self.check(self.lib.frehg_resident_use(self.h, C.byref(n), C.byref(g), C.byref(c), C.byref(b)))
+        return n.value, g.value, c.value, b.value
 
 
 def _fp(a):

@@ -354,6 +354,12 @@ int frehg_profile_reset(frehg_ctx_t ctx);
  * frehg_re_init. CG on operators of up to about a million rows runs whole in one launch instead (no
  * SpMV launches, and none to time) unless a shape is pinned. No counterpart in the reference (PETSc's MatMult has no launch shape). */
 int frehg_spmv_shape(frehg_ctx_t ctx, int precision, int* cells_per_lane, int* kchunk);
+/* This context's CG solves that ran whole in one launch since it was created: launches, those of
+ * them that gave up because their blocks were not all on the device at once (other processes or
+ * streams held a part of it; the solve is then done by the streaming kernels, and after a
+ * pause of up to 64 solves the next one is tried as one launch again), and cells per thread and
+ * blocks of the last one. Any pointer may be null. No counterpart in the reference. */
+int frehg_resident_use(frehg_ctx_t ctx, int64_t* launches, int64_t* gave_up, int* cells_per_thread, int* blocks);
 /* Streaming probe on `device`: the CG SpMV's HBM access mix (six FP64 reads and two FP64 writes
  * per cell, 16-byte accesses) with no neighbours and no reduction, over eight arrays of `cells`
  * doubles that it allocates and frees; for each of a few grid sizes, `reps` timed launches after
