@@ -16,10 +16,12 @@
 //   update: x += alpha y + omega z, r = s - omega t, partials rh.r, ||D^-1 r||^2;
 //                                                fin: convergence test, beta, rho
 #include <algorithm>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 #include "cg_resident.hpp"
@@ -1267,11 +1269,6 @@ void Krylov::build() {
   FREHG_HIP(hipStreamSynchronize(s_));
 }
 
-Krylov::~Krylov() {
-  resident_leave();
-  release();
-}
-
 void Krylov::release() {
   if (borrowed_) return;  // the workspace belongs to the caller
   for (void* p : {(void*)r_, (void*)z_, (void*)p0_, (void*)p1_, (void*)q_, (void*)xw_, (void*)b32_,
@@ -1507,15 +1504,43 @@ int Krylov::cg_outcome(double* res_norm, double* rhs_norm, bool* converged) {
 }
 
 namespace {
-// Launches of the resident solver with more than one block wait for one another's blocks, so two of
-// them (on two contexts' streams) must not share a device. Per device: the stream of the last such launch;
-// a launch on another stream first waits until that one has drained.
+// Launches of the resident solver with more than one block wait for one another's blocks, so two of them (on two
+// contexts' streams) had better not share a device: the contexts of a process take turns, from the launch until
+// its own thread has seen the outcome. A turn is not waited for longer than a launch waits for its blocks (the
+// gates then keep the launches apart), nor kept by a thread that never came back for the outcome. The other
+// context's stream is left alone: it may be capturing, and neither waiting for it nor for an event recorded on it
+// earlier is allowed then.
 constexpr int kMaxDevices = 64;
+using TurnClock = std::chrono::steady_clock;
 struct ResidentTurn {
   std::mutex mu;
-  hipStream_t last = nullptr;
-  const void* owner = nullptr;
+  const void* holder = nullptr;
+  TurnClock::time_point since;
 } g_resident[kMaxDevices];
+
+void turn_take(int device, const void* who) {
+  ResidentTurn& turn = g_resident[device % kMaxDevices];
+  const auto t0 = TurnClock::now();
+  for (;;) {
+    const auto now = TurnClock::now();
+    {
+      std::lock_guard<std::mutex> lock(turn.mu);
+      if (!turn.holder || turn.holder == who || now - turn.since > std::chrono::milliseconds(100)) {
+        turn.holder = who;
+        turn.since = now;
+        return;
+      }
+    }
+    if (now - t0 > std::chrono::microseconds(kCgGateTicks / 100)) return;
+    std::this_thread::yield();
+  }
+}
+
+void turn_give(int device, const void* who) {
+  ResidentTurn& turn = g_resident[device % kMaxDevices];
+  std::lock_guard<std::mutex> lock(turn.mu);
+  if (turn.holder == who) turn.holder = nullptr;
+}
 
 template <typename T, bool THREE_D>
 void launch_resident(int cpt, unsigned int nblk, size_t lds, hipStream_t s, const CgResidentArgs<T>& a) {
@@ -1574,15 +1599,8 @@ void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T
   a.gate_ticks = gate_ticks_;
   a.wait_ticks = wait_ticks_;
   a.launch = launch_;
-  std::unique_lock<std::mutex> lock;
-  if (pl.nblk > 1) {
-    ResidentTurn& turn = g_resident[device_ % kMaxDevices];
-    lock = std::unique_lock<std::mutex>(turn.mu);
-    if (turn.last && turn.last != s_) FREHG_HIP(hipStreamSynchronize(turn.last));
-    turn.last = s_;
-    turn.owner = this;
-  }
   multi_ = pl.nblk > 1;
+  if (multi_) turn_take(device_, this);
   use_->launches += 1;
   use_->cells_per_thread = pl.cpt;
   use_->blocks = (int)pl.nblk;
@@ -1594,6 +1612,7 @@ void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T
 // solves as the last time twice, up to 64, so that waiting in vain (5 ms) stays a small part of the time, and a
 // device that is free again is used again.
 bool Krylov::resident_ended() {
+  if (multi_) turn_give(device_, this);
   if (host_ctl_[1].iters == 0) {
     failed_dirty_ = !host_ctl_->converged;
     if (multi_) use_->pause = 0;
@@ -1605,13 +1624,9 @@ bool Krylov::resident_ended() {
   return false;
 }
 
-void Krylov::resident_leave() {
-  ResidentTurn& turn = g_resident[device_ % kMaxDevices];
-  std::lock_guard<std::mutex> lock(turn.mu);
-  if (turn.owner != this) return;
-  (void)hipStreamSynchronize(s_);
-  turn.last = nullptr;
-  turn.owner = nullptr;
+Krylov::~Krylov() {
+  if (multi_) turn_give(device_, this);  // (an outcome that was never looked at)
+  release();
 }
 
 template <typename T>

@@ -178,7 +178,6 @@ class Krylov {
                        bool guard, double rtol, double atol, int max_it, const T* r0, const KrylovCtl* started);
   bool resident_ended();
   bool resident_turn(int prec);  // resident(), counting a skipped turn
-  void resident_leave();
   // The launch, and the wait for it.
   template <typename T>
   bool cg_resident(const StencilView<T>& A, const T* b, const T* bn, T* x, const unsigned char* fixed, bool zero,
