@@ -55,12 +55,14 @@ struct NaOperator {
 
 // Every entry of the padded operator, right-hand side and iterate: interior rows from the owned
 // arrays (3D rows z-fastest, 2D rows x-fastest), zero elsewhere (ghosts, pitch padding, faces on
-// the domain edge). flags: bit 0 = a +face coupling differs from its neighbour's -face coupling
-// (CG needs a symmetric operator), bit 1 = a zero or non-finite diagonal.
+// the domain edge). flags (pinned host memory): word 0 is set to 1 when a +face coupling differs from its
+// neighbour's -face coupling (CG needs a symmetric operator), word 1 at a zero or non-finite diagonal.
 // (the operators of one-block resident solves and of 2D; larger 3D ones take k_na_pack3). *failed is the word
 // that the solve sets for the unpack kernel; a bad row sets it too, unless this kernel is the one to clear it.
 __device__ inline void na_bad(int* flags, int* failed, int bad) {
-  __hip_atomic_fetch_or(flags, bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);  // pinned host memory
+  // (plain stores: the bus has no atomic OR on host memory)
+  if (bad & 1) __hip_atomic_store(&flags[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (bad & 2) __hip_atomic_store(&flags[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   if (failed) __hip_atomic_store(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __global__ __launch_bounds__(NT) void k_na_pack(Geo g, int three, NaOperator op, long long n, double* D, double* ax,
@@ -150,7 +152,7 @@ __global__ __launch_bounds__(NT) void k_na_pack3(Geo g, NaOperator op, double* D
 // x to the owned order, unless the solve before failed.
 __global__ __launch_bounds__(NT) void k_na_unpack(Geo g, int three, const double* x, double* x_owned,
                                                   const int* failed, const int* flags) {
-  if ((failed && *failed) || (flags && *flags)) return;
+  if ((failed && *failed) || (flags && (flags[0] || flags[1]))) return;
   const int nz = three ? g.nz : 1;
   const long long r = (long long)blockIdx.x * NT + threadIdx.x;
   if (r >= (long long)g.nx * g.ny * nz) return;
@@ -181,7 +183,7 @@ void noalloc_setup(int device) {
   const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
   if (e != hipSuccess || ptr == nullptr)
     throw HipError(std::string("hipGetSymbolAddress(scratch) failed: ") + hipGetErrorString(e));
-  // results of a call, written by its kernels: two control blocks and the flag word (held, as the scratch
+  // results of a call, written by its kernels: two control blocks and the flag words (held, as the scratch
   // array is, until the process ends)
   void* host = nullptr;
   if (hipHostMalloc(&host, 3 * sizeof(KrylovCtl), hipHostMallocDefault) != hipSuccess || host == nullptr)
@@ -230,8 +232,8 @@ void ls_solve_noalloc(int device, hipStream_t s, int ndim, int nx, int ny, int n
   (void)take(sizeof(int));
   KrylovWorkspace ws = Krylov::carve_workspace(base, g, three);
   ws.host = g_host_ctl[device];
-  int* flags = &ws.host[2].iters;
-  *flags = 0;
+  int* flags = reinterpret_cast<int*>(&ws.host[2]);  // two words behind the control blocks
+  flags[0] = flags[1] = 0;
   Profiler off;  // no timing events (they would be created on first use)
   Krylov kry(g, three, s, &off, use, ws);
   NaOperator op{};
@@ -269,9 +271,8 @@ void ls_solve_noalloc(int device, hipStream_t s, int ndim, int nx, int ny, int n
   const bool queued = kry.enqueue(A, b, nullptr, x, nullptr, true, kc);
   if (queued) unpack(kry.failed_flag());
   FREHG_HIP(hipStreamSynchronize(s));
-  const int hflags = *flags;
-  if (hflags & 2) throw ArgError("frehg_ls_solve_noalloc: zero diagonal (Jacobi needs D != 0)");
-  if (hflags & 1) throw ArgError("frehg_ls_solve_noalloc: operator is not symmetric (CG requires A = A^T)");
+  if (flags[1]) throw ArgError("frehg_ls_solve_noalloc: zero diagonal (Jacobi needs D != 0)");
+  if (flags[0]) throw ArgError("frehg_ls_solve_noalloc: operator is not symmetric (CG requires A = A^T)");
   SolveResult sr;
   if (!queued || !kry.finish_queued(&sr)) {
     if (queued) zero(ws.r, ws.ctl + 3);  // the exchange buffers become CG vectors again

@@ -118,3 +118,22 @@ def test_noalloc_leaves_the_solution_alone_on_a_bad_operator(ndim, nx, ny, nz):
         x, st = _solve_noalloc(ctx, ndim, nx, ny, nz, diag, offs, b, cfg)
         assert st.converged
         np.testing.assert_allclose(x, ref, rtol=0, atol=1e-8 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("ndim,nx,ny,nz", [(3, 33, 5, 65), (2, 45, 50, 1), (3, 9, 8, 7)])
+def test_noalloc_reports_both_faults_of_an_operator(ndim, nx, ny, nz):
+    """A zero diagonal and a nonsymmetric coupling of rows far apart, found by different blocks of the pack kernel: the
+    diagonal is what the call names, whichever is found first; each alone is named by the call after."""
+    ctx = gpu.Context(0)
+    diag, offs, b = spd_stencil(ndim, nx, ny, nz, 6)
+    cfg = abi.solver_config(1e-11)
+    d, o = diag.copy(), [v.copy() for v in offs]
+    o[1][0] *= 1.5
+    for faults, what in (((1, 1), "diagonal"), ((1, 0), "diagonal"), ((0, 1), "symmetric"), ((1, 1), "diagonal")):
+        d[-1] = 0.0 if faults[0] else diag[-1]
+        o[1][0] = offs[1][0] * (1.5 if faults[1] else 1.0)
+        with pytest.raises(gpu.FrehgError) as e:
+            _solve_noalloc(ctx, ndim, nx, ny, nz, d, o, b, cfg)
+        assert e.value.code == abi.ERR_INVALID_ARG and what in str(e.value)
+    x, st = _solve_noalloc(ctx, ndim, nx, ny, nz, diag, offs, b, cfg)
+    assert st.converged
