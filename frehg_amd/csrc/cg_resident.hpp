@@ -66,6 +66,8 @@ struct CgResidentArgs {
   const KrylovCtl* ctl;      // and its control block
   KrylovCtl* out;            // result (device or pinned host memory)
   int* gave_up;              // set to 1 when a wait ends without its word
+  int* refused;              // null, or a device word: not 0 on entry when the operator is not to be solved (one
+                             // block: cleared again)
   int* failed;               // device word for kernels queued behind: set to 1 unless the solve converges
   double rtol, atol;
   int max_it, guard, x0_zero;
@@ -216,6 +218,8 @@ __global__ __launch_bounds__(kCgNT) void k_cg_resident(CgResidentArgs<T> P) {
     }
     return;
   }
+  const int refused =
+      P.refused ? __hip_atomic_load(P.refused, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;  // (used below)
   if (tid == 0) {
     dead = 0;
     bound = P.wait_ticks;
@@ -339,6 +343,14 @@ __global__ __launch_bounds__(kCgNT) void k_cg_resident(CgResidentArgs<T> P) {
       if (tid == 0) cg_give_up(P.gave_up, P.failed);
       return;
     }
+  }
+
+  if (refused) {
+    if (first) {
+      if (nblk == 1) *P.refused = 0;
+      cg_fail(P.failed);
+    }
+    return;
   }
 
   // Pause between posting and the first look, in units of 64 clocks: a look that comes too early costs

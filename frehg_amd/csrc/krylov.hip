@@ -1577,6 +1577,7 @@ void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T
   host_ctl_[1].iters = 0;
   a.out = out;
   a.gave_up = &out[1].iters;
+  a.refused = refused_;
   a.failed = failed_flag();
   if (failed_dirty_ && !borrowed_) FREHG_HIP(hipMemsetAsync(a.failed, 0, sizeof(int), s_));  // (borrowed: cleared)
   failed_dirty_ = true;  // until its outcome has been seen
@@ -1639,9 +1640,11 @@ bool Krylov::cg_resident(const StencilView<T>& A, const T* b, const T* bn, T* x,
 }
 
 bool Krylov::enqueue(const StencilView<double>& A, const double* b, const double* bn, double* x,
-                     const unsigned char* fixed, bool x0_zero, const KrylovConfig& cfg) {
+                     const unsigned char* fixed, bool x0_zero, const KrylovConfig& cfg, int* refused) {
   if (cfg.ksp != FREHG_KSP_CG || cfg.precision != 0 || !host_out_ || !resident(0) || !A.symmetric()) return false;  // (solve() counts a skipped turn)
+  refused_ = refused;
   resident_launch<double>(A, b, bn, x, fixed, x0_zero, false, cfg.rtol, cfg.atol, cfg.max_it, nullptr, nullptr);
+  refused_ = nullptr;
   return true;
 }
 

@@ -132,12 +132,15 @@ class Krylov {
   // solve() without the wait, where the solve is one launch (FP64 CG on a resident-size operator): queues
   // it and returns true, or returns false and does nothing. After the stream has drained, finish_queued gives
   // the outcome as solve() would (it throws as solve() does), or false when the solve has to be done again
-  // with solve() (x holds a mixture of iterates) together with the work queued behind it.
+  // with solve() (x holds a mixture of iterates) together with the work queued behind it. refused (may be null): a
+  // device word that a kernel queued before has set when the operator is not to be solved; the solve then ends at
+  // once as failed, without an outcome.
   bool enqueue(const StencilView<double>& A, const double* b, const double* bn, double* x, const unsigned char* fixed,
-               bool x0_zero, const KrylovConfig& cfg);
+               bool x0_zero, const KrylovConfig& cfg, int* refused = nullptr);
   bool finish_queued(SolveResult* res);
   // Device word that a queued solve sets to 1 unless it converges, for the kernels queued behind it.
   int* failed_flag() const { return &ctl_[2].iters; }
+  int* refused_flag() const { return &ctl_[2].max_it; }  // room for such a word
 
   // CG SpMV launch shape per precision (0 FP64, 1 FP32): cells per lane (1: one column per
   // thread on 64 x 4 tiles; 2: two adjacent columns per lane on 128 x 4 tiles, paired aligned
@@ -259,6 +262,7 @@ class Krylov {
   unsigned long long *halo_[4] = {}, *mail_ = nullptr;  // its exchange buffers: low, low, high, high words; sums
   size_t mail_words_ = 0;
   long long gate_ticks_ = kCgGateTicks, wait_ticks_ = kCgWaitTicks;
+  int* refused_ = nullptr;        // of the solve being queued
   bool multi_ = false;            // the last resident launch had several blocks
   int last_iters_ = 8;
   int last_inner_iters_ = 8;

@@ -29,6 +29,8 @@
 // process ends). Host code never passes its name to a kernel or a copy: the name is a host-side
 // stand-in, and the device address comes from hipGetSymbolAddress (scratch_ptr_).
 static __device__ __align__(256) unsigned char scratch[frehg::kScratchBytes];
+// Set by the pack kernel of a one-block solve whose operator is not to be solved, cleared by that solve.
+static __device__ int one_refused;
 
 namespace frehg {
 
@@ -37,6 +39,7 @@ namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_setup_mu;
 void* g_scratch_ptr[kMaxDevices] = {};  // device address of `scratch`, per device
+int* g_refused_ptr[kMaxDevices] = {};  // device address of `one_refused`, per device
 KrylovCtl* g_host_ctl[kMaxDevices] = {};  // pinned results of a call, per device
 std::mutex g_call_mu[kMaxDevices];      // serialises this process's calls per device
 
@@ -57,16 +60,19 @@ struct NaOperator {
 // arrays (3D rows z-fastest, 2D rows x-fastest), zero elsewhere (ghosts, pitch padding, faces on
 // the domain edge). flags (pinned host memory): word 0 is set to 1 when a +face coupling differs from its
 // neighbour's -face coupling (CG needs a symmetric operator), word 1 at a zero or non-finite diagonal.
-// (the operators of one-block resident solves and of 2D; larger 3D ones take k_na_pack3). *failed is the word
-// that the solve sets for the unpack kernel; a bad row sets it too, unless this kernel is the one to clear it.
-__device__ inline void na_bad(int* flags, int* failed, int bad) {
+// (the operators of one-block resident solves and of 2D; larger 3D ones take k_na_pack3). A bad row also sets
+// *refused, at which the solve queued behind ends at once, and *failed, the word that the solve sets for the unpack
+// kernel, unless this kernel is the one to clear it (the solve then sets it).
+__device__ inline void na_bad(int* flags, int* refused, int* failed, int bad) {
   // (plain stores: the bus has no atomic OR on host memory)
   if (bad & 1) __hip_atomic_store(&flags[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   if (bad & 2) __hip_atomic_store(&flags[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(refused, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (failed) __hip_atomic_store(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __global__ __launch_bounds__(NT) void k_na_pack(Geo g, int three, NaOperator op, long long n, double* D, double* ax,
-                                                double* ay, double* az, double* b, double* x, int* flags, int* failed, int clear) {
+                                                double* ay, double* az, double* b, double* x, int* flags,
+                                                int* refused, int* failed, int clear) {
   if (clear && blockIdx.x == 0 && threadIdx.x == 0) *failed = 0;
   const long long c = (long long)blockIdx.x * NT + threadIdx.x;
   if (c >= n) return;
@@ -97,7 +103,7 @@ __global__ __launch_bounds__(NT) void k_na_pack(Geo g, int three, NaOperator op,
     vx = plus(0, ii < g.nx - 1, three ? r + nz : r + 1);
     vy = plus(1, j < g.ny - 1, three ? r + (long long)g.nx * nz : r + g.nx);
     if (three) vz = plus(2, k < nz - 1, r + 1);
-    if (bad) na_bad(flags, clear ? nullptr : failed, bad);
+    if (bad) na_bad(flags, refused, clear ? nullptr : failed, bad);
   }
   D[c] = d;
   ax[c] = vx;
@@ -112,7 +118,7 @@ __global__ __launch_bounds__(NT) void k_na_pack(Geo g, int three, NaOperator op,
 // took 74 us at 128 x 96 x 48 (each 64-byte line of the eight inputs fetched once per layer it holds).
 constexpr int kPt = 32;
 __global__ __launch_bounds__(NT) void k_na_pack3(Geo g, NaOperator op, double* D, double* ax, double* ay, double* az,
-                                                 double* b, int* flags, int* failed) {
+                                                 double* b, int* flags, int* refused, int* failed) {
   __shared__ double lds[5][kPt][kPt + 1];
   const int j = blockIdx.x, i0 = blockIdx.y * kPt, k0 = blockIdx.z * kPt;
   const int u = threadIdx.x & (kPt - 1), v0 = threadIdx.x / kPt;
@@ -135,7 +141,7 @@ __global__ __launch_bounds__(NT) void k_na_pack3(Geo g, NaOperator op, double* D
     lds[3][u][v] = plus(2, k < g.nz - 1, r + 1);
     lds[4][u][v] = op.b[r];
   }
-  if (bad) na_bad(flags, failed, bad);
+  if (bad) na_bad(flags, refused, failed, bad);
   __syncthreads();
   for (int v = v0; v < kPt; v += NT / kPt) {
     const int i = i0 + u, k = k0 + v;
@@ -151,8 +157,8 @@ __global__ __launch_bounds__(NT) void k_na_pack3(Geo g, NaOperator op, double* D
 
 // x to the owned order, unless the solve before failed.
 __global__ __launch_bounds__(NT) void k_na_unpack(Geo g, int three, const double* x, double* x_owned,
-                                                  const int* failed, const int* flags) {
-  if ((failed && *failed) || (flags && (flags[0] || flags[1]))) return;
+                                                  const int* failed) {
+  if (failed && *failed) return;
   const int nz = three ? g.nz : 1;
   const long long r = (long long)blockIdx.x * NT + threadIdx.x;
   if (r >= (long long)g.nx * g.ny * nz) return;
@@ -183,6 +189,11 @@ void noalloc_setup(int device) {
   const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
   if (e != hipSuccess || ptr == nullptr)
     throw HipError(std::string("hipGetSymbolAddress(scratch) failed: ") + hipGetErrorString(e));
+  void* word = nullptr;
+  const hipError_t e1 = hipGetSymbolAddress(&word, HIP_SYMBOL(one_refused));
+  if (e1 != hipSuccess || word == nullptr)
+    throw HipError(std::string("hipGetSymbolAddress(one_refused) failed: ") + hipGetErrorString(e1));
+  g_refused_ptr[device] = static_cast<int*>(word);
   // results of a call, written by its kernels: two control blocks and the flag words (held, as the scratch
   // array is, until the process ends)
   void* host = nullptr;
@@ -245,6 +256,7 @@ void ls_solve_noalloc(int device, hipStream_t s, int ndim, int nx, int ny, int n
   // units, they are exchange buffers whose words must not carry a tag) with the control blocks behind
   // them. A resident solve of one block exchanges nothing.
   const bool one = kry.resident_blocks(0) == 1, tiled = three && !one;
+  int* refused = one ? g_refused_ptr[device] : kry.refused_flag();
   auto zero = [&](double* from, void* to) {
     const long long zn = (reinterpret_cast<char*>(to) - reinterpret_cast<char*>(from)) / (long long)sizeof(double);
     hipLaunchKernelGGL(k_na_zero, dim3((unsigned)std::min<long long>(4096, (zn + NT - 1) / NT)), dim3(NT), 0, s, from,
@@ -254,21 +266,21 @@ void ls_solve_noalloc(int device, hipStream_t s, int ndim, int nx, int ny, int n
   if (!one) zero(tiled ? D : ws.r, ws.ctl + 3);
   if (tiled)
     hipLaunchKernelGGL(k_na_pack3, dim3(ny, ceil_div(nx, kPt), ceil_div(nz, kPt)), dim3(NT), 0, s, g, op, D, ax, ay, az,
-                       b, flags, kry.failed_flag());
+                       b, flags, refused, kry.failed_flag());
   else
     hipLaunchKernelGGL(k_na_pack, dim3(ceil_div(n, NT)), dim3(NT), 0, s, g, three ? 1 : 0, op, n, D, ax, ay, az, b, x,
-                       flags, kry.failed_flag(), one ? 1 : 0);
+                       flags, refused, kry.failed_flag(), one ? 1 : 0);
   FREHG_LAUNCH_CHECK();
   const StencilView<double> A{D, ax, ay, az};
   const long long rows = (long long)nx * ny * (three ? nz : 1);
   auto unpack = [&](const int* failed) {
     hipLaunchKernelGGL(k_na_unpack, dim3(ceil_div(rows, NT)), dim3(NT), 0, s, g, three ? 1 : 0, (const double*)x,
-                       x_owned, failed, failed && one ? flags : nullptr);
+                       x_owned, failed);
     FREHG_LAUNCH_CHECK();
   };
   // A one-launch solve is queued with the unpack kernel behind it and the call waits once; the checks of the
   // operator are looked at before the solve's outcome, so they are reported as before.
-  const bool queued = kry.enqueue(A, b, nullptr, x, nullptr, true, kc);
+  const bool queued = kry.enqueue(A, b, nullptr, x, nullptr, true, kc, refused);
   if (queued) unpack(kry.failed_flag());
   FREHG_HIP(hipStreamSynchronize(s));
   if (flags[1]) throw ArgError("frehg_ls_solve_noalloc: zero diagonal (Jacobi needs D != 0)");

@@ -137,3 +137,44 @@ def test_noalloc_reports_both_faults_of_an_operator(ndim, nx, ny, nz):
         assert e.value.code == abi.ERR_INVALID_ARG and what in str(e.value)
     x, st = _solve_noalloc(ctx, ndim, nx, ny, nz, diag, offs, b, cfg)
     assert st.converged
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(13, 12, 13), (40, 41, 30), (128, 60, 40)])
+def test_noalloc_refuses_without_solving(nx, ny, nz):
+    """An operator that CG takes long over (couplings over many decades, hardly any storage, tolerances that are never
+    met) is refused for one nonsymmetric entry in a small part of the time of its symmetric form."""
+    import time
+    rng = np.random.default_rng(9)
+    diag, offs, b = spd_stencil(3, nx, ny, nz, 6)
+    diag = 1e-12 * np.ones(nx * ny * nz)
+    n = np.arange(nx * ny * nz)
+    for d, s in ((0, nz), (1, nx * nz), (2, 1)):
+        p = offs[2 * d + 1]
+        p[:] = np.where(p != 0.0, -np.exp(4.0 * rng.standard_normal(p.size)), 0.0)
+        offs[2 * d][:] = 0.0
+        rows = n[p != 0.0]
+        offs[2 * d][rows + s] = p[rows]
+    for a in offs:
+        diag -= a
+    cfg = abi.solver_config(0.0, atol=0.0, max_it=4000)
+    ctx = gpu.Context(0)
+    seconds = []
+    for asym in (False, True, False, True):
+        o = [v.copy() for v in offs]
+        if asym:
+            o[3][np.flatnonzero(o[3])[-1]] *= 1.5
+        dd, oo, bb = _dev(diag), [_dev(v) for v in o], _dev(b)
+        x = torch.full_like(bb, 7.0)
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        try:
+            ctx.ls_solve_noalloc(3, nx, ny, nz, dd.data_ptr(), [v.data_ptr() for v in oo], bb.data_ptr(),
+                                 x.data_ptr(), cfg)
+        except gpu.FrehgError as e:
+            assert ("symmetric" in str(e)) == asym
+        else:
+            assert not asym
+        seconds.append(time.perf_counter() - t0)
+    print(f"{nx}x{ny}x{nz}: solved in {seconds[2] * 1e3:.2f} ms, refused in {seconds[3] * 1e3:.2f} ms")
+    assert seconds[2] > 2e-3, "the case must keep CG busy"
+    assert seconds[3] < 0.25 * seconds[2]
