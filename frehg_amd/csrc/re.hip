@@ -619,7 +619,7 @@ void ReState::set_params(const frehg_re_params& p) {
   const bool first = (dtn_ == 0.0);
   p_ = p;
   kc_fresh_ = false;
-  skip_check_ = 0;
+  checks_.clear();
   if (first) dtn_ = p.dt;
 }
 
@@ -742,7 +742,7 @@ void ReState::set_initial(const double* h_int, const double* wc_int) {
   FREHG_HIP(hipStreamSynchronize(s_));
   dtn_ = p_.dt;
   inc_valid_ = false;
-  skip_check_ = 0;
+  checks_.clear();
 }
 
 void ReState::learned_increment(double* dst) {
@@ -1049,9 +1049,7 @@ void ReState::step(frehg_re_stats* st) {
     // system is stored and solved at once, and the solve's first sweep is the test. At 512x512x30 a
     // failed test costs 275 us of a 2.7 ms step; a test that would have passed and was not taken costs
     // 190 us once (assembly with sweep and the fluxes alone, 483 us, against 275 us with both).
-    const unsigned int bit = m < 32 ? 1u << m : 0u;
-    const bool expect_fail = (skip_check_ & bit) != 0;
-    const bool spec = !zero && picard_check_ && m < p_.picard_max && !expect_fail;
+    const bool spec = !zero && picard_check_ && m < p_.picard_max && !checks_.expect_fail(m);
     if (spec) {
       hipEvent_t ev0 = check_flux_ ? prof_->start(FREHG_KT_GW_CORRECT) : nullptr;
       hipEvent_t ev1 = check_flux_ ? prof_->stop() : nullptr;
@@ -1081,12 +1079,13 @@ void ReState::step(frehg_re_stats* st) {
       // here the passes at h^m = h^{m-1} have repeated their results
       local.picard_converged = 1;
       flux_done = spec && check_flux_;
-      skip_check_ &= ~(m - 1 < 32 ? 1u << (m - 1) : 0u);
+      checks_.ended(m - 1);
       break;
     }
     if (hres_[0] <= p_.picard_tol) {
       local.picard_converged = 1;
       flux_done = spec && check_flux_;
+      checks_.ended(m);
       break;
     }
     if (m >= p_.picard_max) break;  // the cap: the step continues from the last iterate
@@ -1101,9 +1100,10 @@ void ReState::step(frehg_re_stats* st) {
         post_done = true;
         flux_done = check_flux_;
         op_pending_ = true;
+        checks_.ended(m);
         break;
       }
-      skip_check_ |= bit;
+      checks_.failed(m);
     }
     // The FP32 copy of the operator is refreshed when the coming solve will need inner solves:
     // from x0 = 0, or after a solve that took a refinement. A solve from h^m that converged at
@@ -1122,7 +1122,7 @@ void ReState::step(frehg_re_stats* st) {
     if (!zero && unchanged) {
       post_done = true;
       local.picard_converged = 1;
-      skip_check_ &= ~bit;
+      checks_.ended(m);
       break;
     }
   }

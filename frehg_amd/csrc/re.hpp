@@ -8,6 +8,7 @@
 #include "../../include/frehg_gpu.h"
 #include "common.hpp"
 #include "krylov.hpp"
+#include "picard_checks.hpp"
 
 namespace frehg {
 
@@ -121,7 +122,7 @@ class ReState {
   // kernels (FREHG_FUSED_START=0: a pass of its own after the start).
   bool fused_start_ = true;
   bool op_pending_ = false;
-  unsigned int skip_check_ = 0;  // bit m: the residual test of iterate h^m failed in the previous step
+  PicardChecks checks_;
   // Both lazy stores, before a change of the state.
   void flush_lazy() {
     materialize_fluxes();
