@@ -47,7 +47,8 @@ KT_SW_SPMV = 5
 KT_SW_UPDATE = 6
 KT_GW_REFINE = 7
 KT_GW_GUESS = 8
-KT_COUNT = 9
+KT_GW_CG = 9
+KT_COUNT = 10
 
 BC_FREE_DRAINAGE = 3
 

@@ -1542,13 +1542,21 @@ void turn_give(int device, const void* who) {
   if (turn.holder == who) turn.holder = nullptr;
 }
 
+template <typename T, bool THREE_D, int CPT>
+void launch_resident_as(unsigned int nblk, size_t lds, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1,
+                        const CgResidentArgs<T>& a) {
+  if (ev0) hipExtLaunchKernelGGL((k_cg_resident<T, THREE_D, CPT>), dim3(nblk), dim3(kCgNT), lds, s, ev0, ev1, 0, a);
+  else hipLaunchKernelGGL((k_cg_resident<T, THREE_D, CPT>), dim3(nblk), dim3(kCgNT), lds, s, a);
+}
+
 template <typename T, bool THREE_D>
-void launch_resident(int cpt, unsigned int nblk, size_t lds, hipStream_t s, const CgResidentArgs<T>& a) {
+void launch_resident(int cpt, unsigned int nblk, size_t lds, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1,
+                     const CgResidentArgs<T>& a) {
   switch (cpt) {
-    case 1: hipLaunchKernelGGL((k_cg_resident<T, THREE_D, 1>), dim3(nblk), dim3(kCgNT), lds, s, a); break;
-    case 2: hipLaunchKernelGGL((k_cg_resident<T, THREE_D, 2>), dim3(nblk), dim3(kCgNT), lds, s, a); break;
-    case 4: hipLaunchKernelGGL((k_cg_resident<T, THREE_D, 4>), dim3(nblk), dim3(kCgNT), lds, s, a); break;
-    default: hipLaunchKernelGGL((k_cg_resident<T, THREE_D, 8>), dim3(nblk), dim3(kCgNT), lds, s, a);
+    case 1: launch_resident_as<T, THREE_D, 1>(nblk, lds, s, ev0, ev1, a); break;
+    case 2: launch_resident_as<T, THREE_D, 2>(nblk, lds, s, ev0, ev1, a); break;
+    case 4: launch_resident_as<T, THREE_D, 4>(nblk, lds, s, ev0, ev1, a); break;
+    default: launch_resident_as<T, THREE_D, 8>(nblk, lds, s, ev0, ev1, a);
   }
   FREHG_LAUNCH_CHECK();
 }
@@ -1605,8 +1613,11 @@ void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T
   use_->launches += 1;
   use_->cells_per_thread = pl.cpt;
   use_->blocks = (int)pl.nblk;
-  if (three_d_) launch_resident<T, true>(pl.cpt, pl.nblk, pl.lds, s_, a);
-  else launch_resident<T, false>(pl.cpt, pl.nblk, pl.lds, s_, a);
+  // (the 2D solves are not timed, as in cg_iterations)
+  hipEvent_t ev0 = three_d_ ? prof_->start(FREHG_KT_GW_CG) : nullptr;
+  hipEvent_t ev1 = three_d_ ? prof_->stop() : nullptr;
+  if (three_d_) launch_resident<T, true>(pl.cpt, pl.nblk, pl.lds, s_, ev0, ev1, a);
+  else launch_resident<T, false>(pl.cpt, pl.nblk, pl.lds, s_, ev0, ev1, a);
 }
 
 // A launch that gave up found the device shared: the next one of the context is tried after as many streamed

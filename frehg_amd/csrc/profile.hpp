@@ -12,7 +12,7 @@
 
 namespace frehg {
 
-constexpr int kKernelTypes = 9;  // FREHG_KT_COUNT
+constexpr int kKernelTypes = 10;  // FREHG_KT_COUNT
 
 // One context's CG solves of one launch (cg_resident.hpp): launches, those that gave up because their blocks were
 // not all on the device, and the tiling of the last one. After a launch that gave up, the next `skip` solves

@@ -337,7 +337,8 @@ enum {
   FREHG_KT_SW_UPDATE = 6,   /* surface Krylov update (reserved, not timed) */
   FREHG_KT_GW_REFINE = 7,   /* groundwater FP64 residual sweep of iterative refinement */
   FREHG_KT_GW_GUESS = 8,    /* learned-guess inference (features + MLP forward) */
-  FREHG_KT_COUNT = 9
+  FREHG_KT_GW_CG = 9,       /* groundwater CG solves that run whole in one launch (FP64 and FP32 inner) */
+  FREHG_KT_COUNT = 10
 };
 int frehg_profile_enable(frehg_ctx_t ctx, int enable);
 /* Kernel types timed while profiling is enabled: bit kt of kernel_mask (default: all). A timed
@@ -351,8 +352,11 @@ int frehg_profile_reset(frehg_ctx_t ctx);
  * FREHG_PREC_MIXED: the FP32 inner solve): cells per lane (1: one column per thread; 2: two
  * adjacent columns per lane with paired aligned loads) and layers per block. Set by the autotuner
  * at the first solve, or pinned by the environment variable FREHG_SPMV_SHAPE="cpl:kchunk" read at
- * frehg_re_init. CG on operators of up to about a million rows runs whole in one launch instead (no
- * SpMV launches, and none to time) unless a shape is pinned. No counterpart in the reference (PETSc's MatMult has no launch shape). */
+ * frehg_re_init. CG on small operators runs whole in one launch instead (timed as FREHG_KT_GW_CG)
+ * unless a shape is pinned: in 3D up to 4 cells per thread of 512 per compute unit, or 8 where
+ * the operator fits the LDS (FP64: about 0.8 million rows on 256 compute units; FP32: about a
+ * million), in 2D up to 4096 rows per compute unit. No counterpart in the reference (PETSc's
+ * MatMult has no launch shape). */
 int frehg_spmv_shape(frehg_ctx_t ctx, int precision, int* cells_per_lane, int* kchunk);
 /* This context's CG solves that ran whole in one launch since it was created: launches, those of
  * them that gave up because their blocks were not all on the device at once (other processes or

@@ -92,3 +92,32 @@ def test_resident_solve_stops_as_the_streaming_one_does():
     assert "breakdown" in str(e.value)
     x, st = ctx.ls_solve(3, 30, 30, 30, diag, offs, np.zeros_like(b), abi.solver_config(1e-10))
     assert st.iterations == 0 and not x.any()
+
+
+@pytest.mark.parametrize("precision", [abi.PREC_FP64, abi.PREC_MIXED])
+def test_profile_times_the_solves_of_one_launch(monkeypatch, precision):
+    """Kernel timing shows the groundwater Krylov work of small grids: whole solves under FREHG_KT_GW_CG, or SpMV
+    and update launches where a shape is pinned."""
+    nx, ny, nz = 30, 22, 15
+    soil = abi.soil_params(alpha=2.0, n=1.8, theta_s=0.40, theta_r=0.05, Ks_x=1e-5, Ks_y=1e-5, Ks_z=1e-5, Ss=1e-5)
+    p = abi.re_params(soil=soil, solver=abi.solver_config(1e-11, precision=precision), dx=0.5, dy=0.5, dz=0.05, dt=30.0,
+                      bc_type=(0, 0, 0, 0, 3, 1), htop=-0.3, adaptive_dt=0, use_full3d=1)
+    for shape in (None, "1:1"):
+        if shape:
+            monkeypatch.setenv("FREHG_SPMV_SHAPE", shape)
+        else:
+            monkeypatch.delenv("FREHG_SPMV_SHAPE", raising=False)
+        ctx = gpu.Context(0)
+        ctx.re_init(nx, ny, nz, p)
+        ctx.re_set_initial(h=np.full(nx * ny * nz, -1.5))
+        ctx.profile_enable(True)
+        ctx.profile_reset()
+        solves = 0
+        for _ in range(3):
+            solves += max(1, ctx.re_step().solve.refinements)
+        cg_ms, cg = ctx.profile_read(abi.KT_GW_CG)
+        streamed = [ctx.profile_read(kt) for kt in (abi.KT_GW_SPMV, abi.KT_GW_SPMV32, abi.KT_GW_UPDATE)]
+        if shape:
+            assert cg == 0 and sum(n for _, n in streamed) >= 2 * solves and sum(ms for ms, _ in streamed) > 0.0
+        else:
+            assert cg == ctx.resident_use()[0] == solves and cg_ms > 0.0 and sum(n for _, n in streamed) == 0
