@@ -1057,8 +1057,8 @@ Krylov::Krylov(const Geo& g, bool three_d, hipStream_t stream, Profiler* prof, R
   part_ = ws.part;
   part_u_ = ws.part_u;
   ctl_ = ws.ctl;
-  host_ctl_ = ws.host ? ws.host : host_ctl_own_;
-  host_out_ = ws.host != nullptr;
+  if (!ws.host) throw ArgError("Krylov: a borrowed workspace needs its pinned control blocks");
+  host_ctl_ = ws.host;
   // the resident solve needs none of the CG vectors: its exchange buffers take their place
   double* words[4] = {r_, z_, p0_, p1_};
   for (int q = 0; q < 4; ++q) halo_[q] = reinterpret_cast<unsigned long long*>(words[q]);
@@ -1580,11 +1580,10 @@ void Krylov::resident_launch(const StencilView<T>& A, const T* b, const T* bn, T
   a.fixed = fixed;
   a.r0 = r0;
   a.ctl = started;
-  // the outcome goes straight to pinned host memory (a borrowed workspace may have none: copied by the caller)
-  KrylovCtl* out = host_out_ ? host_ctl_ : ctl_;
+  // the outcome goes straight to pinned host memory
   host_ctl_[1].iters = 0;
-  a.out = out;
-  a.gave_up = &out[1].iters;
+  a.out = host_ctl_;
+  a.gave_up = &host_ctl_[1].iters;
   a.refused = refused_;
   a.failed = failed_flag();
   if (failed_dirty_ && !borrowed_) FREHG_HIP(hipMemsetAsync(a.failed, 0, sizeof(int), s_));  // (borrowed: cleared)
@@ -1645,14 +1644,13 @@ template <typename T>
 bool Krylov::cg_resident(const StencilView<T>& A, const T* b, const T* bn, T* x, const unsigned char* fixed, bool zero,
                          bool guard, double rtol, double atol, int max_it, const T* r0, const KrylovCtl* started) {
   resident_launch<T>(A, b, bn, x, fixed, zero, guard, rtol, atol, max_it, r0, started);
-  if (!host_out_) FREHG_HIP(hipMemcpyAsync(host_ctl_, ctl_, 2 * sizeof(KrylovCtl), hipMemcpyDeviceToHost, s_));
   FREHG_HIP(hipStreamSynchronize(s_));
   return resident_ended();
 }
 
 bool Krylov::enqueue(const StencilView<double>& A, const double* b, const double* bn, double* x,
                      const unsigned char* fixed, bool x0_zero, const KrylovConfig& cfg, int* refused) {
-  if (cfg.ksp != FREHG_KSP_CG || cfg.precision != 0 || !host_out_ || !resident(0) || !A.symmetric()) return false;  // (solve() counts a skipped turn)
+  if (cfg.ksp != FREHG_KSP_CG || cfg.precision != 0 || !resident(0) || !A.symmetric()) return false;  // (solve() counts a skipped turn)
   refused_ = refused;
   resident_launch<double>(A, b, bn, x, fixed, x0_zero, false, cfg.rtol, cfg.atol, cfg.max_it, nullptr, nullptr);
   refused_ = nullptr;

@@ -52,7 +52,7 @@ struct KrylovWorkspace {
   double *r = nullptr, *z = nullptr, *p0 = nullptr, *p1 = nullptr, *q = nullptr;
   double *part = nullptr, *part_u = nullptr;
   KrylovCtl* ctl = nullptr;
-  KrylovCtl* host = nullptr;  // two pinned host control blocks (optional: one-launch solves can then be queued)
+  KrylovCtl* host = nullptr;  // two control blocks in pinned host memory
   long long n = 0;
 };
 
@@ -251,10 +251,8 @@ class Krylov {
   double* part_ = nullptr;
   double* stage_ = nullptr;  // first-stage sums of a caller's sweep partials (5 x kRedStage)
   KrylovCtl* ctl_ = nullptr;  // [0] main / outer, [1] inner
-  KrylovCtl* host_ctl_ = nullptr;
-  bool host_out_ = true;   // host_ctl_ is pinned: launches write their outcome to it
+  KrylovCtl* host_ctl_ = nullptr;  // two, pinned: one-launch solves write their outcome and whether they gave up
   bool borrowed_ = false;  // workspace owned by the caller (no allocation, no autotuning)
-  KrylovCtl host_ctl_own_[2] = {};  // host mirrors of the control blocks in borrowed mode
   ResidentPlan plan_[2];          // resident CG solve per precision (0 FP64, 1 FP32)
   int device_ = 0;
   bool failed_dirty_ = true;      // failed_flag() may hold a failure
