@@ -1146,8 +1146,10 @@ void Krylov::setup_shapes() {
 
 // Tiling of the resident CG solve: a solve of up to 2048 rows takes one block (no exchange), a larger one
 // the fewest cells per thread (1, 2, 4, 8) whose tiles number at most one per compute unit, and of those the
-// tiling with the least halo and blocks. Operators beyond eight cells per thread (4096 rows per compute
-// unit, fewer where the LDS is short) stream: there an iteration is bound by HBM, not by latency.
+// tiling with the least halo and blocks. Operators beyond eight cells per thread stream: there an iteration is
+// bound by HBM, not by latency. Eight cells are 4096 rows per compute unit (1.05 million on 256) in 2D and in
+// FP32; a 3D operator in FP64 takes 40 B and more per cell of LDS beside the halo of p, which holds about
+// 3400 rows (100 x 90 x 90 runs in one launch, 101 x 100 x 100 streams).
 // us per iteration on MI355X, streaming (at the shapes the solver chose) and resident:
 //   rows    819   4096   8000   80000  131072  262144 (3D)  512000  589824 | 2D: 2400  16384  262144  360000
 //   stream  28.1  34.7   40.0   67.7   51.6    90.0         93.3    75.7   |     20.5  20.4   25.4    28.7

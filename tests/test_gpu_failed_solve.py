@@ -51,3 +51,30 @@ def test_failed_queued_solve_leaves_the_fields(monkeypatch, lazy, picard, guess)
         # of the iterate itself the fields of the failed step's unconverged head differ by far more
         scale = np.abs(b[f]).max()
         assert np.abs(a[f] - b[f]).max() <= 1e-9 * scale, f
+
+
+@pytest.mark.parametrize("nx,ny", [(40, 45), (150, 97)])  # one block, several
+def test_failed_surface_solve_leaves_the_fields(monkeypatch, nx, ny):
+    """The same of a surface step, whose kernels behind the solve are queued with it."""
+    say(f"failed surface solve: {nx}x{ny}")
+    rng = np.random.default_rng(8)
+    bed, depth = 0.1 * rng.random((ny, nx)), 0.3 + 0.2 * rng.random((ny, nx))
+    fields = []
+    for shape in (None, "1:1"):
+        if shape:
+            monkeypatch.setenv("FREHG_SPMV_SHAPE", shape)
+        else:
+            monkeypatch.delenv("FREHG_SPMV_SHAPE", raising=False)
+        ctx = gpu.Context(0)
+        ctx.swe_init(nx, ny, 1.0, 1.0, abi.swe_params(manning=0.03, dt=1.0, solver=abi.solver_config(1e-12, max_it=3)))
+        ctx.swe_set_bathymetry(bed.ravel())
+        ctx.swe_set_initial_eta((bed + depth).ravel())
+        with pytest.raises(gpu.FrehgError) as e:
+            ctx.swe_step(1e-5)
+        assert e.value.code == abi.ERR_NOT_CONVERGED
+        assert (ctx.resident_use()[0] == 1) == (shape is None)
+        fields.append({f: ctx.swe_get(f) for f in abi.SWE_FIELDS})
+    for f in abi.SWE_FIELDS:
+        a, b = (v[f] for v in fields)
+        # (three iterations from the same start in another order of sums)
+        assert np.abs(a - b).max() <= 1e-9 * max(1.0, np.abs(b).max()), f
