@@ -1,8 +1,8 @@
 // Whole Jacobi-CG solves in one launch, with the solve's vectors resident on the compute units.
 //
-// For operators of up to about a million rows (see Krylov::resident_plan) an iteration moves so little that the two kernels of
-// the streaming solver (k_spmv, k_cg_update) are bound by their launches and by the time a few blocks
-// take to fill. Here each block keeps a box of the grid for the whole solve: x, z = D^-1 r, D and the
+// For operators of up to about a million rows (see Krylov::resident_plan) an iteration moves so little that
+// the two kernels of the streaming solver (k_spmv, k_cg_update) are bound by their launches and by the time a
+// few blocks take to fill. Here each block keeps a box of the grid for the whole solve: x, z = D^-1 r, D and the
 // couplings of its cells in registers, p with a one-cell halo in LDS. Nothing but one value per halo cell
 // and five partial sums leave a block per iteration, and no memory is streamed inside the loop.
 //

@@ -6,11 +6,10 @@ import json
 import os
 import subprocess
 import sys
-import time
+import threading
 
 import numpy as np
 import pytest
-import torch
 
 from frehg_amd import abi, gpu, workloads
 from gpu_common import say
@@ -143,6 +142,8 @@ def processes(tmp_path, n):
     outs = [str(tmp_path / f"out{n}_{k}.npz") for k in range(n)]
     ps = [subprocess.Popen([sys.executable, str(child), o], stdin=subprocess.PIPE, stdout=subprocess.PIPE, text=True)
           for o in outs]
+    watchdog = threading.Timer(90.0, lambda: [p.kill() for p in ps])  # (a read below has no time limit of its own)
+    watchdog.start()
     try:
         for p in ps:
             assert p.stdout.readline().strip() == "ready"
@@ -151,6 +152,7 @@ def processes(tmp_path, n):
             p.stdin.flush()
         res = [json.loads(p.communicate(timeout=60)[0].splitlines()[-1]) for p in ps]
     finally:
+        watchdog.cancel()
         for p in ps:
             if p.poll() is None:
                 p.kill()
